@@ -83,6 +83,7 @@ struct BatchArgs {
   int* t_fill;
   V* a_w;
   V* t_w;
+  double *a_s, *t_s;  // FP64 scaled values: a_w and t_w themselves in FP64
   // unscaled problem (minimisation form)
   const double* c;
   const double* lb;
@@ -443,68 +444,40 @@ struct BScaleEpi {
   __device__ void row(int r, const Acc& s, const Pre&, double (&)[kMaxRed]) const { out[r] = s.value(); }
 };
 
-// Power iteration on the FP64 scaled matrix, values formed on the fly as in
-// the scaled copy of the single-LP solver: A~^T q, then A~ (A~^T q).
-struct BPowerAtEpi {
+// One product of the power iteration or Lanczos over a scaled FP64 matrix: A~^T q, or
+// A~ (A~^T q) with the power iteration's q . (A~ A~^T q).  `vec` is gathered (through
+// LdsGather or GlobalGather, which read it through a typed pointer), out is one
+// value per row; both are LDS or global memory, by LP.  Each step was bound by its
+// gathers: forming ((a D_r) D_c) (z / ||z||) per nonzero took two gathers and an FP64
+// division; reading the scaled values that the loop uses anyway (and a copy of them
+// in FP64 for FP32-mixed), with z / ||z|| formed once per row, leaves one gather.
+// The terms and their order are unchanged.  512 LPs in FP64 (m 50 to 2 000):
+// 278.6 -> 240.7 ms a call; 1 024 LPs in FP32-mixed: 128.5 -> 125.7 ms.
+template <class Out>
+struct BSpmvEpi {
   using Mat = double;
   using Acc = AccSum64;
   struct Pre {};
-  const double* Dr;
-  const double* Dc;
-  const double* z;
-  double nrm;
-  double* atq;
-  __device__ double product(double v, int col, int r) const { return ((v * Dc[r]) * Dr[col]) * (z[col] / nrm); }
+  Out out;
   __device__ Pre load(int) const { return Pre{}; }
-  __device__ void row(int r, const Acc& s, const Pre&, double (&)[kMaxRed]) const { atq[r] = s.value(); }
+  __device__ void row(int r, const Acc& s, const Pre&, double (&)[kMaxRed]) const { out[r] = s.value(); }
 };
+template <class Q>
 struct BPowerAEpi {
   using Mat = double;
   using Acc = AccSum64;
   struct Pre {
-    double zold;
+    double q;
   };
-  const double* Dr;
-  const double* Dc;
-  const double* atq;
-  const double* zold;
-  double nrm;
-  double* znew;
-  __device__ double product(double v, int col, int r) const { return ((v * Dr[r]) * Dc[col]) * atq[col]; }
-  __device__ Pre load(int r) const { return Pre{zold[r]}; }
+  Q q;
+  __attribute__((address_space(1))) double* znew;
+  __device__ Pre load(int r) const { return Pre{q[r]}; }
   __device__ void row(int r, const Acc& sum, const Pre& p, double (&red)[kMaxRed]) const
   {
     const double s = sum.value();
     znew[r]        = s;
-    red[0] += (p.zold / nrm) * s;
+    red[0] += p.q * s;
   }
-};
-
-// Lanczos on A~ A~^T (FP32-mixed): A~^T q, then A~ (A~^T q), FP64 values formed
-// on the fly in the operand order of the scaled copies.
-struct BLzAtEpi {
-  using Mat = double;
-  using Acc = AccSum64;
-  struct Pre {};
-  const double* Dr;
-  const double* Dc;
-  const double* q;
-  double* atq;
-  __device__ double product(double v, int col, int r) const { return ((v * Dc[r]) * Dr[col]) * q[col]; }
-  __device__ Pre load(int) const { return Pre{}; }
-  __device__ void row(int r, const Acc& s, const Pre&, double (&)[kMaxRed]) const { atq[r] = s.value(); }
-};
-struct BLzAEpi {
-  using Mat = double;
-  using Acc = AccSum64;
-  struct Pre {};
-  const double* Dr;
-  const double* Dc;
-  const double* atq;
-  double* z;
-  __device__ double product(double v, int col, int r) const { return ((v * Dr[r]) * Dc[col]) * atq[col]; }
-  __device__ Pre load(int) const { return Pre{}; }
-  __device__ void row(int r, const Acc& s, const Pre&, double (&)[kMaxRed]) const { z[r] = s.value(); }
 };
 
 // Largest eigenvalue of the symmetric tridiagonal matrix of k Lanczos steps,
@@ -710,10 +683,22 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     __syncthreads();
   }
   // scaled working matrices, reference operand order (vals * first[row]) * second[col]
+  // (and, in FP32-mixed, the FP64 ones that Lanczos reads; in FP64 they are the same arrays)
+  constexpr bool kF32 = std::is_same<V, float>::value;
+  double* as64 = A.a_s + d.nz0;
+  double* ts64 = A.t_s + d.nz0;
   for (int i = tid; i < m; i += kBT)
-    for (int k = aptr[i]; k < aptr[i + 1]; ++k) aw[k] = (V)((aorig[k] * Dr[i]) * Dc[aidx[k]]);
+    for (int k = aptr[i]; k < aptr[i + 1]; ++k) {
+      const double v = (aorig[k] * Dr[i]) * Dc[aidx[k]];
+      as64[k]        = v;
+      if constexpr (kF32) aw[k] = (V)v;
+    }
   for (int j = tid; j < n; j += kBT)
-    for (int k = tptr[j]; k < tptr[j + 1]; ++k) tw[k] = (V)((torig[k] * Dc[j]) * Dr[tidx[k]]);
+    for (int k = tptr[j]; k < tptr[j + 1]; ++k) {
+      const double v = (torig[k] * Dc[j]) * Dr[tidx[k]];
+      ts64[k]        = v;
+      if constexpr (kF32) tw[k] = (V)v;
+    }
   // vectors and norms (bound_objective_rescaling)
   zero_red(red);
   for (int j = tid; j < n; j += kBT) {
@@ -748,13 +733,31 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   }
   double s2  = 0.0;
   int piters = 0;
-  if constexpr (std::is_same<V, float>::value) {
+  // ---- step size.  q and A~^T q, the vectors its products gather, live in LDS at
+  // the end of the dynamic LDS (the loop's vectors are not in use yet) when a
+  // single-buffered stage fits before them.
+  const long long pvec_off = (lds_bytes - (long long)(m + n) * (long long)sizeof(double)) & ~15LL;
+  const bool pin           = pvec_off >= (long long)kStage * 12;
+  double* qv  = pin ? reinterpret_cast<double*>(dyn_lds + pvec_off) : pz;
+  double* atq = pin ? qv + m : patq;
+  st.dbl8     = 2LL * kStage * 12 <= (pin ? pvec_off : lds_bytes);
+  using LdsOut  = __attribute__((address_space(3))) double*;
+  using GlobOut = __attribute__((address_space(1))) double*;
+  auto at_pass  = [&]() {  // atq = A~^T q
+    if (pin) {
+      using E = BSpmvEpi<LdsOut>;
+      rows_pass(tptr, tidx, ts64, d.lgt, tblk, st, LdsGather<E>{E{(LdsOut)atq}, as_lds((const double*)qv)}, red);
+    } else {
+      using E = BSpmvEpi<GlobOut>;
+      rows_pass(tptr, tidx, ts64, d.lgt, tblk, st, GlobalGather<E>{E{(GlobOut)atq}, as_global((const double*)qv)}, red);
+    }
+  };
+  if constexpr (kF32) {
     // ---- FP32-mixed: Lanczos on A~ A~^T, as the single-LP solver's
     // lanczos_sigma_max_sq (hashed start, at most 240 steps, stop when the Ritz
     // value moves by at most 1e-6 relative or beta^2 vanishes).  Scratch vectors
-    // not yet in use: q, q_prev in pz / pz2, w in rowv (scaling is done), A~ A~^T q
+    // not yet in use: q_prev in pz2, w in rowv (scaling is done), A~ A~^T q
     // in yu (first written by the first termination check).
-    double* q  = pz;
     double* qp = pz2;
     double* w  = rowv;
     double* zb = yu;
@@ -762,34 +765,35 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     zero_red(red);
     for (int i = tid; i < m; i += kBT) {
       const double v = hashed_start(i);
-      q[i]           = v;
+      qv[i]          = v;
       qp[i]          = 0.0;
       red[0] += v * v;
     }
     wg_sum<1>(red, lds);
     const double inv = 1.0 / sqrt(red[0]);
-    for (int i = tid; i < m; i += kBT) q[i] = q[i] * inv;
+    for (int i = tid; i < m; i += kBT) qv[i] = qv[i] * inv;
     __syncthreads();
     const int kmax = min(m, kLzMax);
     double theta = 0.0, prev = -1.0;
     while (piters < kmax) {
       const int j = piters;
       zero_red(red);
-      rows_pass(tptr, tidx, torig, d.lgt, tblk, st, BLzAtEpi{Dr, Dc, q, patq}, red);
-      __syncthreads();
-      rows_pass(aptr, aidx, aorig, d.lga, ablk, st, BLzAEpi{Dr, Dc, patq, zb}, red);
+      at_pass();
+      using E = BSpmvEpi<GlobOut>;
+      if (pin) rows_pass(aptr, aidx, as64, d.lga, ablk, st, LdsGather<E>{E{(GlobOut)zb}, as_lds((const double*)atq)}, red);
+      else rows_pass(aptr, aidx, as64, d.lga, ablk, st, GlobalGather<E>{E{(GlobOut)zb}, as_global((const double*)atq)}, red);
       const double bp = j > 0 ? sqrt(ab[2 * j - 1]) : 0.0;
       zero_red(red);
       for (int i = tid; i < m; i += kBT) {
         const double v = zb[i] - bp * qp[i];
         w[i]           = v;
-        red[0] += q[i] * v;
+        red[0] += qv[i] * v;
       }
       wg_sum<1>(red, lds);
       const double alpha = red[0];
       zero_red(red);
       for (int i = tid; i < m; i += kBT) {
-        const double v = w[i] - alpha * q[i];
+        const double v = w[i] - alpha * qv[i];
         w[i]           = v;
         red[0] += v * v;
       }
@@ -807,42 +811,48 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       if (stop) break;
       const double sb = sqrt(b2);
       for (int i = tid; i < m; i += kBT) {
-        qp[i] = q[i];
-        q[i]  = w[i] / sb;
+        qp[i] = qv[i];
+        qv[i] = w[i] / sb;
       }
       __syncthreads();
     }
     s2 = theta;
   } else {
-    // ---- power iteration (compute_initial_step_size, pdlp.cu:2622-2738)
-    for (int i = tid; i < m; i += kBT) pz[i] = A.z0[i];
+    // ---- power iteration (compute_initial_step_size, pdlp.cu:2622-2738); qv holds z / ||z||
+    double* zn = pz2;
     zero_red(red);
     for (int i = tid; i < m; i += kBT) red[0] += A.z0[i] * A.z0[i];
     wg_sum<1>(red, lds);
     double nrm = sqrt(red[0]);
-    double* zo = pz;
-    double* zn = pz2;
+    for (int i = tid; i < m; i += kBT) qv[i] = A.z0[i] / nrm;
+    __syncthreads();
     while (piters < 5000) {
       zero_red(red);
-      rows_pass(tptr, tidx, torig, d.lgt, tblk, st, BPowerAtEpi{Dr, Dc, zo, nrm, patq}, red);
-      __syncthreads();
-      rows_pass(aptr, aidx, aorig, d.lga, ablk, st, BPowerAEpi{Dr, Dc, patq, zo, nrm, zn}, red);
+      at_pass();
+      if (pin) {
+        using E = BPowerAEpi<const __attribute__((address_space(3))) double*>;
+        rows_pass(aptr, aidx, as64, d.lga, ablk, st,
+                  LdsGather<E>{E{as_lds((const double*)qv), (GlobOut)zn}, as_lds((const double*)atq)}, red);
+      } else {
+        using E = BPowerAEpi<const __attribute__((address_space(1))) double*>;
+        rows_pass(aptr, aidx, as64, d.lga, ablk, st,
+                  GlobalGather<E>{E{as_global((const double*)qv), (GlobOut)zn}, as_global((const double*)atq)}, red);
+      }
       wg_sum<1>(red, lds);
       s2 = red[0];
       zero_red(red);
       for (int i = tid; i < m; i += kBT) {
-        const double q = zo[i] / nrm;
-        const double r = q * -s2 + zn[i];
+        const double z = zn[i];
+        const double r = qv[i] * -s2 + z;
         red[0] += r * r;
-        red[1] += zn[i] * zn[i];
+        red[1] += z * z;
       }
       wg_sum<2>(red, lds);
       ++piters;
       if (sqrt(red[0]) < 1e-4) break;
       nrm = sqrt(red[1]);
-      double* t = zo;
-      zo        = zn;
-      zn        = t;
+      for (int i = tid; i < m; i += kBT) qv[i] = zn[i] / nrm;
+      __syncthreads();
     }
   }
   const double eta = 0.998 / sqrt(s2);
@@ -1316,6 +1326,9 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
   auto colv = arena.take<double>(N);
   auto a_w = arena.take<V>(Zp);
   auto t_w = arena.take<V>(Zp);
+  constexpr bool kF32 = std::is_same<V, float>::value;
+  auto a_s = arena.take<double>(kF32 ? Zp : 1);
+  auto t_s = arena.take<double>(kF32 ? Zp : 1);
   auto c_w = arena.take<V>(N);
   auto x0 = arena.take<V>(N);
   auto x1 = arena.take<V>(N);
@@ -1434,6 +1447,8 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
   args.t_fill = t_fill.get();
   args.a_w = a_w.get();
   args.t_w = t_w.get();
+  args.a_s = kF32 ? a_s.get() : reinterpret_cast<double*>(a_w.get());
+  args.t_s = kF32 ? t_s.get() : reinterpret_cast<double*>(t_w.get());
   args.c = c.get();
   args.lb = lb.get();
   args.ub = ub.get();
