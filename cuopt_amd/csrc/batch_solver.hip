@@ -24,6 +24,7 @@
 // row epilogue.
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <condition_variable>
 #include <cmath>
 #include <cstring>
@@ -43,11 +44,29 @@ namespace cuopt_amd {
 
 namespace {
 
-constexpr int kBT = 256;  // lanes per LP workgroup
-// Workgroups per CU the kernel is built for (its register budget, __launch_bounds__)
-// and the LDS share of each.  Three (at most 168 VGPRs) spilled ~100 registers
-// to scratch and ran 10-40 % slower than two.
-constexpr int kWgPerCu = 2;
+// Lanes per LP workgroup: a narrow workgroup of kRef lanes, two to a CU, or a wide one
+// of kWide lanes with a CU of its own and all of its LDS, so that every gathered
+// vector fits.  One LP takes about 0.55 times as long per iteration when wide (m 1 200 to
+// 2 000: FP32-mixed 75.7 -> 47.1 us, FP64 132.6 -> 82.8 us; 512 lanes 48.1 / 86.4 us), but
+// it takes twice the share of the chip.  With few LPs the largest ones set the time of
+// the launch and with many the sum does, so the host picks the width by the
+// estimate of both (prefer_wide): 1 024 LPs of m 50 to 2 000 in FP32-mixed 119 ->
+// 75 ms, 512 in FP64 188 -> 117 ms with wide ones; 4 096 in FP32-mixed 216 ms narrow
+// against 252 ms.  LPs of fewer than kWideNnz nonzeros are narrow in any batch
+// (9 us per iteration either way).
+//
+// Every reduction over an LP is summed in the order of kRef lanes (lane v holds the
+// terms v, v + kRef, ... of an elementwise sum, and in a row pass those of the rows
+// that lane v owns in the row blocks of a kRef-lane workgroup), whatever the width:
+// an LP's result does not depend on the workgroup that solves it, bit for bit.
+constexpr int kRef     = 256;
+constexpr int kWide    = 768;
+constexpr int kWideNnz = 2000;
+
+// Workgroups per CU that a width is built for (its register budget,
+// __launch_bounds__, and the LDS share of each).  Three narrow ones (at most 168
+// VGPRs) spilled ~100 registers to scratch and ran 10-40 % slower than two.
+constexpr int wg_per_cu(int bt) { return bt == kRef ? 2 : 1; }
 
 struct BatchDesc {
   int m, n, nnz;
@@ -56,6 +75,8 @@ struct BatchDesc {
   int lga, lgt;       // log2 lanes per row for A and A^T
   int ablk0, nablk;   // row blocks of A: start rows at blk[ablk0 .. ablk0 + nablk]
   int tblk0, ntblk;   // row blocks of A^T
+  int aref0, naref;   // row blocks of A and A^T for kRef lanes: the order of the reductions
+  int tref0, ntref;   // (the same blocks in a narrow workgroup)
   long long nz0;      // offset in nonzero arrays
   double obj_sf, obj_off;
 };
@@ -113,6 +134,7 @@ struct BatchArgs {
   // LPs than resident workgroups, later LPs start later, so the launch can take
   // longer than the limit (at most about the number of dispatch waves times it).
   unsigned long long tick_limit;
+  double* red_rows;               // wide workgroups: the reduction terms of a row pass, by row (4 per row and column)
   double* lz;                     // FP32-mixed: Lanczos coefficients, kLzStride per LP (by LP index)
   const int* blk;                 // row-block starts of every LP's A and A^T (plan_row_blocks)
   int lds_bytes;                  // dynamic LDS of the launch: the stage, then the gathered vectors
@@ -143,34 +165,26 @@ __device__ inline bool check_at(long long k)
 
 // ---- workgroup reductions (fixed order) -------------------------------------
 
-// x holds the same value in every lane: say so to the compiler, which then keeps
-// it (and what is computed from it: the restart and termination scalars) in
-// scalar registers instead of one vector register pair per value.
-__device__ inline double uniform_d(double x)
-{
-  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b & 0xffffffffu));
-  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
+// Sums of the first kRef lanes' values (the others hold none), in every lane.
 template <int NR>
 __device__ inline void wg_sum(double (&v)[kMaxRed], double (*lds)[kMaxRed])
 {
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  if (wid < kRef / kWave) {
 #pragma unroll
-  for (int k = 0; k < NR; ++k)
+    for (int k = 0; k < NR; ++k)
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, kWave);
-  if (lane == 0)
+      for (int off = kWave / 2; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, kWave);
+    if (lane == 0)
 #pragma unroll
-    for (int k = 0; k < NR; ++k) lds[wid][k] = v[k];
+      for (int k = 0; k < NR; ++k) lds[wid][k] = v[k];
+  }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NR; ++k) {
     double s = lds[0][k];
-    for (int w = 1; w < kBT / kWave; ++w) s += lds[w][k];
-    v[k] = uniform_d(s);
+    for (int w = 1; w < kRef / kWave; ++w) s += lds[w][k];
+    v[k] = uniform_value(s);
   }
   __syncthreads();
 }
@@ -184,7 +198,7 @@ __device__ inline void zero_red(double (&r)[kMaxRed])
 // ---- row passes ---------------------------------------------------------------
 
 // Row passes walk an LP's CSR in row blocks planned on the host (plan_row_blocks):
-// a block holds at most kBlockNnz nonzeros and at most one row per lane group,
+// a block holds at most block_nnz nonzeros and at most one row per lane group,
 // or is a single row longer than that.  The stage has two buffers; block b uses
 // buffer b & 1.  While the workgroup reduces block b from LDS it
 //   - copies block b + 1's indices / values into the other buffer with
@@ -194,24 +208,29 @@ __device__ inline void zero_red(double (&r)[kMaxRed])
 // Each group of G lanes reduces one row and runs the epilogue.
 // Each lane adds its row's products in increasing k and groups merge by a
 // fixed shuffle tree, so the sums do not depend on the blocking.
-constexpr int kStage      = 2560;                // entries per stage buffer
-constexpr int kBlockNnz   = kStage - 8;          // nonzeros per staged block (room for the copy's slack)
-constexpr int kStageBytes = 2 * kStage * 12;     // two buffers of 8-byte values and 4-byte indices
+constexpr int stage_len(int bt) { return bt == kRef ? 2560 : 5120; }  // entries per stage buffer
+constexpr int kLongRow = stage_len(kRef) - 8;    // a longer row is a block of its own, read in place
+// nonzeros per staged block (room for the copy's slack)
+constexpr int block_nnz(int bt) { return stage_len(bt) - 8; }
+constexpr int stage_bytes(int bt) { return 2 * stage_len(bt) * 12; }  // two buffers of 8-byte values and 4-byte indices
 constexpr int kNnzPad     = 4;                   // extra elements after each nonzero array (16 bytes or more)
 
 // The stage occupies the start of the workgroup's dynamic LDS.  A pass over
 // values of VB bytes (8 for the FP64 matrices, 4 for FP32 working ones) lays
-// out its buffers by VB: values of buffer b at base + b * kStage * VB, then the
+// out its buffers by VB: values of buffer b at base + b * stage_len * VB, then the
 // indices; it double-buffers when dbl8 / dbl4 says the two buffers fit.
 struct Stage {
   unsigned char* base;
-  uint64_t* merge;  // kBT / kWave accumulator slots
+  uint64_t* merge;  // kRef / kWave accumulator slots
+  double* red_rows; // reduction terms by row (wide workgroups)
   bool dbl8, dbl4;  // two buffers for passes over 8- / 4-byte values
 };
 
 struct RowBlocks {
   const int* start;  // first row of each block; start[nblk] = number of rows
   int nblk;
+  const int* ref;    // the same for kRef lanes
+  int nref;
 };
 
 // Lanes per row and row blocks of one matrix (rows given by their lengths).
@@ -225,16 +244,16 @@ int plan_lanes(int nrows, long long nnz)
 }
 
 template <class Len>
-void plan_row_blocks(int nrows, int lg, Len len, std::vector<int>& out)
+void plan_row_blocks(int nrows, int lg, int lanes, Len len, std::vector<int>& out)
 {
-  const int max_rows = kBT >> lg;
+  const int max_rows = lanes >> lg, max_nnz = block_nnz(lanes);
   int r              = 0;
   out.push_back(0);
   while (r < nrows) {
     long long z = len(r);
     int e       = r + 1;
-    if (z <= kBlockNnz)
-      while (e < nrows && e - r < max_rows && z + len(e) <= kBlockNnz) z += len(e++);
+    if (z <= kLongRow)
+      while (e < nrows && e - r < max_rows && len(e) <= kLongRow && z + len(e) <= max_nnz) z += len(e++);
     out.push_back(e);
     r = e;
   }
@@ -250,10 +269,11 @@ __device__ inline int dword_mis(const void* p)
 // at the 16-byte boundary at or below src + d0, so dword d0 lands at
 // dst[dword_mis(src + d0)], and up to 3 dwords past d1 come along (the nonzero
 // arrays carry kNnzPad elements of padding).  Wave w moves pieces
-// w*64 + i*256 + lane; global_load_lds with 16 bytes writes lane l's piece to
+// w*64 + i*BT + lane; global_load_lds with 16 bytes writes lane l's piece to
 // the wave-uniform LDS address given plus 16 l.  One 16-byte request moves four
 // times the data of a dword request, and the copy is bound by requests.  The
 // caller's barrier waits for it.
+template <int BT>
 __device__ inline void copy_to_lds(const int* __restrict__ src, long long d0, long long d1, int* dst)
 {
   if (d1 <= d0) return;
@@ -261,133 +281,31 @@ __device__ inline void copy_to_lds(const int* __restrict__ src, long long d0, lo
   const int mis  = dword_mis(src + d0);
   const int* s0  = src + d0 - mis;
   const int npc  = (int)((d1 - d0 + mis + 3) >> 2);
-  for (int base = w * kWave; base < npc; base += kBT)
+  for (int base = w * kWave; base < npc; base += BT)
     if (base + lane < npc)
       __builtin_amdgcn_global_load_lds(s0 + 4 * (base + lane), dst + 4 * base, 16, 0, 0);
 }
 
-// Fixed-order workgroup merge of one accumulator (wave butterflies, then waves 0..3).
+// Fixed-order workgroup merge of the first kRef lanes' accumulators (wave
+// butterflies, then waves 0..3).
 template <class Acc>
 __device__ inline Acc wg_merge(Acc a, uint64_t* slots)
 {
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  if (wid < kRef / kWave) {
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) a.merge(a.shfl(off));
-  if (lane == 0) slots[wid] = a.pack();
+    for (int off = kWave / 2; off > 0; off >>= 1) a.merge(a.shfl(off));
+    if (lane == 0) slots[wid] = a.pack();
+  }
   __syncthreads();
   Acc r = Acc::unpack(slots[0]);
-  for (int w = 1; w < kBT / kWave; ++w) r.merge(Acc::unpack(slots[w]));
+  for (int w = 1; w < kRef / kWave; ++w) r.merge(Acc::unpack(slots[w]));
   __syncthreads();
   return r;
 }
 
-// Rows [0, nrows) of one LP's CSR; Epi as in spmv_tiles.hpp, with the row index
-// passed as the third argument of product().
-template <class Epi>
-__device__ inline void rows_pass(const int* __restrict__ ptr,
-                                 const int* __restrict__ idx,
-                                 const typename Epi::Mat* __restrict__ vals,
-                                 int lg,
-                                 RowBlocks blocks,
-                                 const Stage& st,
-                                 const Epi& epi,
-                                 double (&red)[kMaxRed])
-{
-  using Acc        = typename Epi::Acc;
-  using Mat        = typename Epi::Mat;
-  using Pre        = typename Epi::Pre;
-  constexpr int W  = (int)(sizeof(Mat) / 4);  // dwords per value
-  constexpr int VB = 4 * W;                   // bytes per staged value
-  const int G = 1 << lg, sub = threadIdx.x & (G - 1), grp = threadIdx.x >> lg;
-  const int nb = blocks.nblk;
-  if (nb <= 0) return;
-  const bool dbl       = W == 1 ? st.dbl4 : st.dbl8;
-  int* const sidx_base = reinterpret_cast<int*>(st.base + (dbl ? 2 : 1) * kStage * VB);
-  // Buffer addresses are computed, not indexed from an array: a runtime-indexed
-  // pointer array would live in scratch, and its load would wait for the copy
-  // in flight.
-  auto stage = [&](int za, int zb, int buf) {
-    copy_to_lds(reinterpret_cast<const int*>(vals), (long long)W * za, (long long)W * zb,
-                reinterpret_cast<int*>(st.base + buf * (kStage * VB)));
-    copy_to_lds(idx, za, zb, sidx_base + buf * kStage);
-  };
-  // (r0, r1) are block bi's rows, (r1, r2) block bi + 1's, z the matching
-  // nonzero offsets; r3 / z3 (block bi + 2's end) are loaded during block bi.
-  int r0 = blocks.start[0], r1 = blocks.start[1];
-  int z0 = ptr[r0], z1 = ptr[r1];
-  int r2 = r1, z2 = z1;
-  if (nb >= 2) {
-    r2 = blocks.start[2];
-    z2 = ptr[r2];
-  }
-  if (dbl && z1 - z0 <= kBlockNnz) stage(z0, z1, 0);
-  // This lane group's row of the current block: its ptr entries and its
-  // epilogue operands, both loaded one block ahead so that the barrier that
-  // waits for a block's copy also covers them.  The loads are clamped into range
-  // instead of guarded, so that no branch waits for them (a wait for a load also
-  // waits for every copy issued before it); a clamped row's operands go unused.
-  auto load_pre = [&](int r, int rend) { return epi.load(min(r, max(rend - 1, 0))); };
-  int pb = ptr[min(r0 + grp, r1)], pe = ptr[min(r0 + grp + 1, r1)];
-  Pre pre = load_pre(r0 + grp, r1);
-  for (int bi = 0; bi < nb; ++bi) {
-    const int cur = dbl ? bi & 1 : 0;
-    // Every wave's copy of block bi has landed (the barrier waits for each
-    // wave's memory operations), and block bi - 1's reads of the other buffer
-    // are done, so it may be refilled.
-    __syncthreads();
-    const int b = pb - z0, e = pe - z0;
-    const int r3          = bi + 3 <= nb ? blocks.start[bi + 3] : r2;
-    const bool stage_next = bi + 1 < nb && z2 - z1 <= kBlockNnz;
-    if (dbl && stage_next) stage(z1, z2, cur ^ 1);
-    if (!dbl && z1 - z0 <= kBlockNnz) {  // one buffer: copy this block now and wait for it
-      stage(z0, z1, 0);
-      __syncthreads();
-    }
-    const int npb = ptr[min(r1 + grp, r2)], npe = ptr[min(r1 + grp + 1, r2)];
-    const Pre npre = load_pre(r1 + grp, r2);
-    if (z1 - z0 > kBlockNnz) {  // one row longer than a block: read it in place (lane 0's pre is row r0's)
-      Acc a = Acc::zero();
-      for (int k = z0 + (int)threadIdx.x; k < z1; k += kBT) a.add(epi.product(vals[k], idx[k], r0));
-      a = wg_merge(a, st.merge);
-      if (threadIdx.x == 0) epi.row(r0, a, pre, red);
-    } else if (r0 + grp < r1) {
-      const int r       = r0 + grp;
-      // where the copy put nonzero z0 (values are 8-byte aligned when W = 2,
-      // so their dword offset is even)
-      const int* sidx  = sidx_base + cur * kStage + dword_mis(idx + z0);
-      const Mat* svals = reinterpret_cast<const Mat*>(st.base + cur * (kStage * VB)) +
-                         dword_mis(reinterpret_cast<const int*>(vals) + (long long)W * z0) / W;
-      Acc a = Acc::zero();
-      int k = b + sub;
-      for (; k + 3 * G < e; k += 4 * G) {  // four LDS reads in flight, added in order
-        const int c0 = sidx[k], c1 = sidx[k + G], c2 = sidx[k + 2 * G], c3 = sidx[k + 3 * G];
-        const Mat v0 = svals[k], v1 = svals[k + G], v2 = svals[k + 2 * G], v3 = svals[k + 3 * G];
-        const auto p0 = epi.product(v0, c0, r), p1 = epi.product(v1, c1, r);
-        const auto p2 = epi.product(v2, c2, r), p3 = epi.product(v3, c3, r);
-        a.add(p0);
-        a.add(p1);
-        a.add(p2);
-        a.add(p3);
-      }
-      for (; k < e; k += G) a.add(epi.product(svals[k], sidx[k], r));
-      for (int off = G >> 1; off > 0; off >>= 1) a.merge(a.shfl(off));
-      if (sub == 0) epi.row(r, a, pre, red);
-    }
-    const int z3 = bi + 3 <= nb ? ptr[r3] : z2;
-    r0 = r1;
-    z0 = z1;
-    r1 = r2;
-    z1 = z2;
-    r2 = r3;
-    z2 = z3;
-    pb  = npb;
-    pe  = npe;
-    pre = npre;
-  }
-  __syncthreads();  // the pass's stores are visible to the whole workgroup
-}
-
-// A PDHG step epilogue whose gathered vector lives in LDS, read through an
+// An epilogue whose product is a times one gathered value, read through a typed
+// pointer: a PDHG step epilogue whose gathered vector lives in LDS, read through an
 // LDS-typed pointer.  Through the generic pointer each gather is a flat load,
 // which the compiler waits for with both counters: one gather in flight at a
 // time, and the first wait of a block also waits for the next block's copy.
@@ -422,6 +340,143 @@ template <typename T>
 __device__ inline const __attribute__((address_space(1))) T* as_global(const T* p)
 {
   return (const __attribute__((address_space(1))) T*)p;
+}
+
+// Rows [0, nrows) of one LP's CSR; Epi as in spmv_tiles.hpp, with the row index
+// passed as the third argument of product().  NR: the epilogue's reductions, each
+// with at most one term per row, left in the first kRef lanes' red for wg_sum.  A
+// wide workgroup, whose lanes own other rows than kRef lanes would, stores the terms
+// by row and adds them up afterwards as those lanes would have.
+template <int BT, int NR, class Epi>
+__device__ inline void rows_pass(const int* __restrict__ ptr,
+                                 const int* __restrict__ idx,
+                                 const typename Epi::Mat* __restrict__ vals,
+                                 int lg,
+                                 RowBlocks blocks,
+                                 const Stage& st,
+                                 const Epi& epi,
+                                 double (&red)[kMaxRed])
+{
+  using Acc        = typename Epi::Acc;
+  using Mat        = typename Epi::Mat;
+  using Pre        = typename Epi::Pre;
+  constexpr int W  = (int)(sizeof(Mat) / 4);  // dwords per value
+  constexpr int VB = 4 * W;                   // bytes per staged value
+  constexpr int kStage = stage_len(BT);
+  const int G = 1 << lg, sub = threadIdx.x & (G - 1), grp = threadIdx.x >> lg;
+  const int nb = blocks.nblk;
+  if (nb <= 0) return;
+  const bool dbl       = W == 1 ? st.dbl4 : st.dbl8;
+  int* const sidx_base = reinterpret_cast<int*>(st.base + (dbl ? 2 : 1) * kStage * VB);
+  // Buffer addresses are computed, not indexed from an array: a runtime-indexed
+  // pointer array would live in scratch, and its load would wait for the copy
+  // in flight.
+  auto stage = [&](int za, int zb, int buf) {
+    copy_to_lds<BT>(reinterpret_cast<const int*>(vals), (long long)W * za, (long long)W * zb,
+                reinterpret_cast<int*>(st.base + buf * (kStage * VB)));
+    copy_to_lds<BT>(idx, za, zb, sidx_base + buf * kStage);
+  };
+  // (r0, r1) are block bi's rows, (r1, r2) block bi + 1's, z the matching
+  // nonzero offsets; r3 / z3 (block bi + 2's end) are loaded during block bi.
+  int r0 = blocks.start[0], r1 = blocks.start[1];
+  int z0 = ptr[r0], z1 = ptr[r1];
+  int r2 = r1, z2 = z1;
+  if (nb >= 2) {
+    r2 = blocks.start[2];
+    z2 = ptr[r2];
+  }
+  auto is_long = [](int ra, int rb, int za, int zb) { return rb - ra == 1 && zb - za > kLongRow; };
+  const int nrows = blocks.start[nb];
+  auto finish = [&](int r, const Acc& a, const Pre& pre) {
+    if constexpr (NR > 0 && BT != kRef) {
+      double t[kMaxRed];
+#pragma unroll
+      for (int k = 0; k < NR; ++k) t[k] = 0.0;
+      epi.row(r, a, pre, t);
+#pragma unroll
+      for (int k = 0; k < NR; ++k) st.red_rows[(size_t)k * nrows + r] = t[k];
+    } else {
+      epi.row(r, a, pre, red);
+    }
+  };
+  if (dbl && !is_long(r0, r1, z0, z1)) stage(z0, z1, 0);
+  // This lane group's row of the current block: its ptr entries and its
+  // epilogue operands, both loaded one block ahead so that the barrier that
+  // waits for a block's copy also covers them.  The loads are clamped into range
+  // instead of guarded, so that no branch waits for them (a wait for a load also
+  // waits for every copy issued before it); a clamped row's operands go unused.
+  auto load_pre = [&](int r, int rend) { return epi.load(min(r, max(rend - 1, 0))); };
+  int pb = ptr[min(r0 + grp, r1)], pe = ptr[min(r0 + grp + 1, r1)];
+  Pre pre = load_pre(r0 + grp, r1);
+  for (int bi = 0; bi < nb; ++bi) {
+    const int cur = dbl ? bi & 1 : 0;
+    // Every wave's copy of block bi has landed (the barrier waits for each
+    // wave's memory operations), and block bi - 1's reads of the other buffer
+    // are done, so it may be refilled.
+    __syncthreads();
+    const int b = pb - z0, e = pe - z0;
+    const int r3          = bi + 3 <= nb ? blocks.start[bi + 3] : r2;
+    const bool stage_next = bi + 1 < nb && !is_long(r1, r2, z1, z2);
+    if (dbl && stage_next) stage(z1, z2, cur ^ 1);
+    if (!dbl && !is_long(r0, r1, z0, z1)) {  // one buffer: copy this block now and wait for it
+      stage(z0, z1, 0);
+      __syncthreads();
+    }
+    const int npb = ptr[min(r1 + grp, r2)], npe = ptr[min(r1 + grp + 1, r2)];
+    const Pre npre = load_pre(r1 + grp, r2);
+    if (is_long(r0, r1, z0, z1)) {  // read it in place (lane 0's pre is row r0's)
+      Acc a = Acc::zero();
+      if (BT == kRef || threadIdx.x < kRef)
+        for (int k = z0 + (int)threadIdx.x; k < z1; k += kRef) a.add(epi.product(vals[k], idx[k], r0));
+      a = wg_merge(a, st.merge);
+      if (threadIdx.x == 0) finish(r0, a, pre);
+    } else if (r0 + grp < r1) {
+      const int r       = r0 + grp;
+      // where the copy put nonzero z0 (values are 8-byte aligned when W = 2,
+      // so their dword offset is even)
+      const int* sidx  = sidx_base + cur * kStage + dword_mis(idx + z0);
+      const Mat* svals = reinterpret_cast<const Mat*>(st.base + cur * (kStage * VB)) +
+                         dword_mis(reinterpret_cast<const int*>(vals) + (long long)W * z0) / W;
+      Acc a = Acc::zero();
+      int k = b + sub;
+      for (; k + 3 * G < e; k += 4 * G) {  // four LDS reads in flight, added in order
+        const int c0 = sidx[k], c1 = sidx[k + G], c2 = sidx[k + 2 * G], c3 = sidx[k + 3 * G];
+        const Mat v0 = svals[k], v1 = svals[k + G], v2 = svals[k + 2 * G], v3 = svals[k + 3 * G];
+        const auto p0 = epi.product(v0, c0, r), p1 = epi.product(v1, c1, r);
+        const auto p2 = epi.product(v2, c2, r), p3 = epi.product(v3, c3, r);
+        a.add(p0);
+        a.add(p1);
+        a.add(p2);
+        a.add(p3);
+      }
+      for (; k < e; k += G) a.add(epi.product(svals[k], sidx[k], r));
+      for (int off = G >> 1; off > 0; off >>= 1) a.merge(a.shfl(off));
+      if (sub == 0) finish(r, a, pre);
+    }
+    const int z3 = bi + 3 <= nb ? ptr[r3] : z2;
+    r0 = r1;
+    z0 = z1;
+    r1 = r2;
+    z1 = z2;
+    r2 = r3;
+    z2 = z3;
+    pb  = npb;
+    pe  = npe;
+    pre = npre;
+  }
+  __syncthreads();  // the pass's stores are visible to the whole workgroup
+  if constexpr (NR > 0 && BT != kRef) {
+    if (threadIdx.x < kRef && sub == 0) {
+      const int v = (int)threadIdx.x >> lg;
+      for (int b = 0; b < blocks.nref; ++b) {
+        const int r = blocks.ref[b] + v;
+        if (r < blocks.ref[b + 1])
+#pragma unroll
+          for (int k = 0; k < NR; ++k) red[k] += st.red_rows[(size_t)k * nrows + r];
+      }
+    }
+    __syncthreads();  // the terms are read before the next pass writes its own
+  }
 }
 
 // Ruiz / Pock-Chambolle statistics of |(a * D_row-side) * D_col-side| in the
@@ -482,10 +537,10 @@ struct BPowerAEpi {
 
 // Largest eigenvalue of the symmetric tridiagonal matrix of k Lanczos steps,
 // ab[2i] = alpha_i (diagonal) and ab[2i+1] = beta_i^2 (squared off-diagonal),
-// by Sturm counts: each round every lane counts the eigenvalues below one of kBT
+// by Sturm counts: each round every lane counts the eigenvalues below one of kRef
 // points spread evenly over the bracket (Gershgorin to start), and the bracket
 // becomes the gap between the last point with fewer than k below and the first
-// with all k below, kBT + 1 times narrower.  Stops at the single-LP solver's
+// with all k below, kRef + 1 times narrower.  Stops at the single-LP solver's
 // bisection tolerance (relative width 1e-15).  Whole workgroup; slot is one LDS int.
 __device__ inline double wg_tridiag_max_eig(const double* ab, int k, int* slot)
 {
@@ -496,40 +551,28 @@ __device__ inline double wg_tridiag_max_eig(const double* ab, int k, int* slot)
     hi = fmax(hi, ab[2 * i] + r);
   }
   for (int round = 0; round < 64 && hi - lo > 1e-15 * fmax(fabs(hi), 1e-300); ++round) {
-    const double step = (hi - lo) / (double)(kBT + 1);
+    const double step = (hi - lo) / (double)(kRef + 1);
     const double x    = lo + step * (double)(threadIdx.x + 1);
     int c             = 0;
     double d          = 1.0;
-    for (int i = 0; i < k; ++i) {
+    for (int i = 0; i < k && threadIdx.x < kRef; ++i) {
       d = ab[2 * i] - x - (i > 0 ? ab[2 * i - 1] / d : 0.0);
       if (d == 0.0) d = -1e-300;
       if (d < 0.0) ++c;
     }
-    if (threadIdx.x == 0) *slot = kBT;
+    if (threadIdx.x == 0) *slot = kRef;
     __syncthreads();
-    if (c >= k) atomicMin(slot, (int)threadIdx.x);
+    if (c >= k && threadIdx.x < kRef) atomicMin(slot, (int)threadIdx.x);
     __syncthreads();
     const int f = *slot;
     __syncthreads();
-    const double nhi = f < kBT ? lo + step * (double)(f + 1) : hi;
+    const double nhi = f < kRef ? lo + step * (double)(f + 1) : hi;
     const double nlo = f > 0 ? lo + step * (double)f : lo;
-    lo               = uniform_d(nlo);
-    hi               = uniform_d(nhi);
+    lo               = uniform_value(nlo);
+    hi               = uniform_value(nhi);
   }
   return hi;
 }
-
-// y = A x (FP64), row index passed to product() as in the other batch passes.
-struct BPlainEpi {
-  using Mat = double;
-  using Acc = AccSum64;
-  struct Pre {};
-  const double* x;
-  double* y;
-  __device__ double product(double v, int col, int) const { return v * x[col]; }
-  __device__ Pre load(int) const { return Pre{}; }
-  __device__ void row(int r, const Acc& s, const Pre&, double (&)[kMaxRed]) const { y[r] = s.value(); }
-};
 
 __device__ inline double bound_sq(double l, double u)
 {
@@ -541,17 +584,20 @@ __device__ inline double bound_sq(double l, double u)
 
 // ---- the kernel ----------------------------------------------------------------
 
-template <typename V>
-__global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> A)
+template <typename V, int BT>
+__global__ __launch_bounds__(BT, wg_per_cu(BT)) void batch_pdlp_kernel(BatchArgs<V> A)
 {
+  constexpr int kStage = stage_len(BT);
   using V2 = typename Vec2<V>::type;
-  __shared__ double lds[kBT / kWave][kMaxRed];
+  __shared__ double lds[kRef / kWave][kMaxRed];
   __shared__ StepScalars sc;
-  __shared__ int scan_lds[kBT];
-  __shared__ uint64_t merge_lds[kBT / kWave];
+  __shared__ int scan_lds[BT];
+  __shared__ uint64_t merge_lds[kRef / kWave];
   extern __shared__ __align__(16) unsigned char dyn_lds[];
   const unsigned long long t_start = wall_clock64();
   const int tid = threadIdx.x;
+  // First index and limit of the elementwise sums, which run on the first kRef lanes.
+  const int sum0 = BT == kRef || tid < kRef ? tid : INT_MAX;
   const BatchDesc d = A.desc[A.order[blockIdx.x]];
   const int m = d.m, n = d.n, nnz = d.nnz;
   // this LP's slices
@@ -589,8 +635,9 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   const long long vec_off   = (lds_bytes - vec_bytes) & ~15LL;
   const bool vec_in_lds     = vec_off >= (long long)kStage * 12;
   const long long region    = vec_in_lds ? vec_off : lds_bytes;  // the stage's LDS in the loop
-  Stage st{dyn_lds, merge_lds, 2LL * kStage * 12 <= lds_bytes, 2LL * kStage * 8 <= lds_bytes};
-  const RowBlocks ablk{A.blk + d.ablk0, d.nablk}, tblk{A.blk + d.tblk0, d.ntblk};
+  Stage st{dyn_lds, merge_lds, A.red_rows + 4 * ((size_t)d.row0 + d.col0), 2LL * kStage * 12 <= lds_bytes, 2LL * kStage * 8 <= lds_bytes};
+  const RowBlocks ablk{A.blk + d.ablk0, d.nablk, A.blk + d.aref0, d.naref},
+    tblk{A.blk + d.tblk0, d.ntblk, A.blk + d.tref0, d.ntref};
   if (vec_in_lds) {
     V* base = reinterpret_cast<V*>(dyn_lds + vec_off);
     ys[0]   = base;
@@ -610,19 +657,19 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   double red[kMaxRed];
 
   // ---- A^T: counting sort by column, then each column segment ordered by source position
-  for (int j = tid; j < n; j += kBT) tfill[j] = 0;
+  for (int j = tid; j < n; j += BT) tfill[j] = 0;
   __syncthreads();
-  for (int k = tid; k < nnz; k += kBT) atomicAdd(&tfill[aidx[k]], 1);
+  for (int k = tid; k < nnz; k += BT) atomicAdd(&tfill[aidx[k]], 1);
   __syncthreads();
   {
-    const int per = (n + kBT - 1) / kBT, j0 = min(n, tid * per), j1 = min(n, j0 + per);
+    const int per = (n + BT - 1) / BT, j0 = min(n, tid * per), j1 = min(n, j0 + per);
     int s = 0;
     for (int j = j0; j < j1; ++j) s += tfill[j];
     scan_lds[tid] = s;
     __syncthreads();
     if (tid == 0) {
       int acc = 0;
-      for (int t = 0; t < kBT; ++t) {
+      for (int t = 0; t < BT; ++t) {
         const int v = scan_lds[t];
         scan_lds[t] = acc;
         acc += v;
@@ -636,17 +683,17 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       tfill[j]    = acc;
       acc += v;
     }
-    if (tid == kBT - 1) tptr[n] = acc;
+    if (tid == BT - 1) tptr[n] = acc;
   }
   __syncthreads();
-  for (int i = tid; i < m; i += kBT)
+  for (int i = tid; i < m; i += BT)
     for (int k = aptr[i]; k < aptr[i + 1]; ++k) {
       const int dst = atomicAdd(&tfill[aidx[k]], 1);
       tpos[dst]     = k;
       tidx[dst]     = i;
     }
   __syncthreads();
-  for (int j = tid; j < n; j += kBT) {  // insertion sort of the (short) column by source position
+  for (int j = tid; j < n; j += BT) {  // insertion sort of the (short) column by source position
     const int b = tptr[j], e = tptr[j + 1];
     for (int p = b + 1; p < e; ++p) {
       const int kp = tpos[p], ip = tidx[p];
@@ -664,22 +711,22 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   __syncthreads();
 
   // ---- Ruiz (x10) and Pock-Chambolle (alpha = 1) equilibration
-  for (int i = tid; i < m; i += kBT) Dr[i] = 1.0;
-  for (int j = tid; j < n; j += kBT) Dc[j] = 1.0;
+  for (int i = tid; i < m; i += BT) Dr[i] = 1.0;
+  for (int j = tid; j < n; j += BT) Dc[j] = 1.0;
   __syncthreads();
   for (int it = 0; it <= 10; ++it) {
     const bool pc = it == 10;
     zero_red(red);
     if (pc) {
-      rows_pass(aptr, aidx, aorig, d.lga, ablk, st, BScaleEpi<false, false>{Dr, Dc, rowv}, red);
-      rows_pass(tptr, tidx, torig, d.lgt, tblk, st, BScaleEpi<true, false>{Dr, Dc, colv}, red);
+      rows_pass<BT, 0>(aptr, aidx, aorig, d.lga, ablk, st, BScaleEpi<false, false>{Dr, Dc, rowv}, red);
+      rows_pass<BT, 0>(tptr, tidx, torig, d.lgt, tblk, st, BScaleEpi<true, false>{Dr, Dc, colv}, red);
     } else {
-      rows_pass(aptr, aidx, aorig, d.lga, ablk, st, BScaleEpi<false, true>{Dr, Dc, rowv}, red);
-      rows_pass(tptr, tidx, torig, d.lgt, tblk, st, BScaleEpi<true, true>{Dr, Dc, colv}, red);
+      rows_pass<BT, 0>(aptr, aidx, aorig, d.lga, ablk, st, BScaleEpi<false, true>{Dr, Dc, rowv}, red);
+      rows_pass<BT, 0>(tptr, tidx, torig, d.lgt, tblk, st, BScaleEpi<true, true>{Dr, Dc, colv}, red);
     }
     __syncthreads();
-    for (int i = tid; i < m; i += kBT) Dr[i] = rowv[i] > 0.0 ? Dr[i] / sqrt(rowv[i]) : Dr[i];
-    for (int j = tid; j < n; j += kBT) Dc[j] = colv[j] > 0.0 ? Dc[j] / sqrt(colv[j]) : Dc[j];
+    for (int i = tid; i < m; i += BT) Dr[i] = rowv[i] > 0.0 ? Dr[i] / sqrt(rowv[i]) : Dr[i];
+    for (int j = tid; j < n; j += BT) Dc[j] = colv[j] > 0.0 ? Dc[j] / sqrt(colv[j]) : Dc[j];
     __syncthreads();
   }
   // scaled working matrices, reference operand order (vals * first[row]) * second[col]
@@ -687,13 +734,13 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   constexpr bool kF32 = std::is_same<V, float>::value;
   double* as64 = A.a_s + d.nz0;
   double* ts64 = A.t_s + d.nz0;
-  for (int i = tid; i < m; i += kBT)
+  for (int i = tid; i < m; i += BT)
     for (int k = aptr[i]; k < aptr[i + 1]; ++k) {
       const double v = (aorig[k] * Dr[i]) * Dc[aidx[k]];
       as64[k]        = v;
       if constexpr (kF32) aw[k] = (V)v;
     }
-  for (int j = tid; j < n; j += kBT)
+  for (int j = tid; j < n; j += BT)
     for (int k = tptr[j]; k < tptr[j + 1]; ++k) {
       const double v = (torig[k] * Dc[j]) * Dr[tidx[k]];
       ts64[k]        = v;
@@ -701,19 +748,19 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     }
   // vectors and norms (bound_objective_rescaling)
   zero_red(red);
-  for (int j = tid; j < n; j += kBT) {
+  for (int j = sum0; j < n; j += kRef) {
     const double cs = c[j] * Dc[j];
     red[0] += cs * cs * 1.0;
     red[1] += c[j] * c[j];
   }
-  for (int i = tid; i < m; i += kBT) {
+  for (int i = sum0; i < m; i += kRef) {
     red[2] += bound_sq(lc[i] * Dr[i], uc[i] * Dr[i]);
     red[3] += bound_sq(lc[i], uc[i]);
   }
   wg_sum<4>(red, lds);
   double beta = 1.0 / (sqrt(red[2]) + 1.0), gamma = 1.0 / (sqrt(red[0]) + 1.0);
   const double b_norm = sqrt(red[3]), c_norm = sqrt(red[1]);
-  for (int j = tid; j < n; j += kBT) {
+  for (int j = tid; j < n; j += BT) {
     const double dc = Dc[j];
     double l = dc == 0.0 ? 0.0 : lb[j] / dc, u = dc == 0.0 ? 0.0 : ub[j] / dc;
     l = l * beta;
@@ -724,7 +771,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     bb.y     = (V)u;
     bnd_w[j] = bb;
   }
-  for (int i = tid; i < m; i += kBT) {
+  for (int i = tid; i < m; i += BT) {
     V2 bb;
     bb.x       = (V)((lc[i] * Dr[i]) * beta);
     bb.y       = (V)((uc[i] * Dr[i]) * beta);
@@ -746,10 +793,10 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   auto at_pass  = [&]() {  // atq = A~^T q
     if (pin) {
       using E = BSpmvEpi<LdsOut>;
-      rows_pass(tptr, tidx, ts64, d.lgt, tblk, st, LdsGather<E>{E{(LdsOut)atq}, as_lds((const double*)qv)}, red);
+      rows_pass<BT, 0>(tptr, tidx, ts64, d.lgt, tblk, st, LdsGather<E>{E{(LdsOut)atq}, as_lds((const double*)qv)}, red);
     } else {
       using E = BSpmvEpi<GlobOut>;
-      rows_pass(tptr, tidx, ts64, d.lgt, tblk, st, GlobalGather<E>{E{(GlobOut)atq}, as_global((const double*)qv)}, red);
+      rows_pass<BT, 0>(tptr, tidx, ts64, d.lgt, tblk, st, GlobalGather<E>{E{(GlobOut)atq}, as_global((const double*)qv)}, red);
     }
   };
   if constexpr (kF32) {
@@ -763,7 +810,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     double* zb = yu;
     double* ab = A.lz + (size_t)A.order[blockIdx.x] * kLzStride;
     zero_red(red);
-    for (int i = tid; i < m; i += kBT) {
+    for (int i = sum0; i < m; i += kRef) {
       const double v = hashed_start(i);
       qv[i]          = v;
       qp[i]          = 0.0;
@@ -771,7 +818,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     }
     wg_sum<1>(red, lds);
     const double inv = 1.0 / sqrt(red[0]);
-    for (int i = tid; i < m; i += kBT) qv[i] = qv[i] * inv;
+    for (int i = tid; i < m; i += BT) qv[i] = qv[i] * inv;
     __syncthreads();
     const int kmax = min(m, kLzMax);
     double theta = 0.0, prev = -1.0;
@@ -780,11 +827,11 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       zero_red(red);
       at_pass();
       using E = BSpmvEpi<GlobOut>;
-      if (pin) rows_pass(aptr, aidx, as64, d.lga, ablk, st, LdsGather<E>{E{(GlobOut)zb}, as_lds((const double*)atq)}, red);
-      else rows_pass(aptr, aidx, as64, d.lga, ablk, st, GlobalGather<E>{E{(GlobOut)zb}, as_global((const double*)atq)}, red);
+      if (pin) rows_pass<BT, 0>(aptr, aidx, as64, d.lga, ablk, st, LdsGather<E>{E{(GlobOut)zb}, as_lds((const double*)atq)}, red);
+      else rows_pass<BT, 0>(aptr, aidx, as64, d.lga, ablk, st, GlobalGather<E>{E{(GlobOut)zb}, as_global((const double*)atq)}, red);
       const double bp = j > 0 ? sqrt(ab[2 * j - 1]) : 0.0;
       zero_red(red);
-      for (int i = tid; i < m; i += kBT) {
+      for (int i = sum0; i < m; i += kRef) {
         const double v = zb[i] - bp * qp[i];
         w[i]           = v;
         red[0] += qv[i] * v;
@@ -792,7 +839,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       wg_sum<1>(red, lds);
       const double alpha = red[0];
       zero_red(red);
-      for (int i = tid; i < m; i += kBT) {
+      for (int i = sum0; i < m; i += kRef) {
         const double v = w[i] - alpha * qv[i];
         w[i]           = v;
         red[0] += v * v;
@@ -810,7 +857,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       prev            = theta;
       if (stop) break;
       const double sb = sqrt(b2);
-      for (int i = tid; i < m; i += kBT) {
+      for (int i = tid; i < m; i += BT) {
         qp[i] = qv[i];
         qv[i] = w[i] / sb;
       }
@@ -821,27 +868,27 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
     // ---- power iteration (compute_initial_step_size, pdlp.cu:2622-2738); qv holds z / ||z||
     double* zn = pz2;
     zero_red(red);
-    for (int i = tid; i < m; i += kBT) red[0] += A.z0[i] * A.z0[i];
+    for (int i = sum0; i < m; i += kRef) red[0] += A.z0[i] * A.z0[i];
     wg_sum<1>(red, lds);
     double nrm = sqrt(red[0]);
-    for (int i = tid; i < m; i += kBT) qv[i] = A.z0[i] / nrm;
+    for (int i = tid; i < m; i += BT) qv[i] = A.z0[i] / nrm;
     __syncthreads();
     while (piters < 5000) {
       zero_red(red);
       at_pass();
       if (pin) {
         using E = BPowerAEpi<const __attribute__((address_space(3))) double*>;
-        rows_pass(aptr, aidx, as64, d.lga, ablk, st,
+        rows_pass<BT, 1>(aptr, aidx, as64, d.lga, ablk, st,
                   LdsGather<E>{E{as_lds((const double*)qv), (GlobOut)zn}, as_lds((const double*)atq)}, red);
       } else {
         using E = BPowerAEpi<const __attribute__((address_space(1))) double*>;
-        rows_pass(aptr, aidx, as64, d.lga, ablk, st,
+        rows_pass<BT, 1>(aptr, aidx, as64, d.lga, ablk, st,
                   GlobalGather<E>{E{as_global((const double*)qv), (GlobOut)zn}, as_global((const double*)atq)}, red);
       }
       wg_sum<1>(red, lds);
       s2 = red[0];
       zero_red(red);
-      for (int i = tid; i < m; i += kBT) {
+      for (int i = sum0; i < m; i += kRef) {
         const double z = zn[i];
         const double r = qv[i] * -s2 + z;
         red[0] += r * r;
@@ -851,7 +898,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       ++piters;
       if (sqrt(red[0]) < 1e-4) break;
       nrm = sqrt(red[1]);
-      for (int i = tid; i < m; i += kBT) qv[i] = zn[i] / nrm;
+      for (int i = tid; i < m; i += BT) qv[i] = zn[i] / nrm;
       __syncthreads();
     }
   }
@@ -862,14 +909,14 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
   st.dbl4 = 2LL * kStage * 8 <= region;
 
   // ---- initial iterates (zeros, projected)
-  for (int j = tid; j < n; j += kBT) {
+  for (int j = tid; j < n; j += BT) {
     const V2 bb = bnd_w[j];
     xhat[j]     = V(0);
     xanc[j]     = V(0);
     xs[0][j]    = mn(mx(V(0), bb.x), bb.y);
     slack[j]    = V(0);
   }
-  for (int i = tid; i < m; i += kBT) {
+  for (int i = tid; i < m; i += BT) {
     yhat[i]  = V(0);
     yanc[i]  = V(0);
     ys[0][i] = V(0);
@@ -894,19 +941,19 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
       // xu carries the gathered primal point until the column pass writes x there.
       const KktPointF<V> point{xhat, Dc, 1.0 / beta, refine_active ? xstar : nullptr, idp, xu};
       double unused[kMaxRed];
-      for (int j = tid; j < n; j += kBT) point(j, unused);
+      for (int j = tid; j < n; j += BT) point(j, unused);
       __syncthreads();
-      rows_pass(aptr, aidx, aorig, d.lga, ablk, st,
-                KktRowsEpi<V>{xu, yhat, Dr, 1.0 / gamma, gamma, cb_orig, yanc, yu, refine_active ? xstar : nullptr,
-                              refine_active ? ystar : nullptr, idp, idd},
-                red);
+      const KktRowsEpi<V> rows{xu, yhat, Dr, 1.0 / gamma, gamma, cb_orig, yanc, yu, refine_active ? xstar : nullptr,
+                               refine_active ? ystar : nullptr, idp, idd};
+      rows_pass<BT, 3>(aptr, aidx, aorig, d.lga, ablk, st,
+                       GlobalGather<KktRowsEpi<V>>{rows, as_global((const double*)xu)}, red);
       wg_sum<3>(red, lds);
       const double rp2 = red[0], psum = red[1], dd = red[2];  // dd: ||y0 - yhat||^2
       zero_red(red);
-      rows_pass(tptr, tidx, torig, d.lgt, tblk, st,
-                KktColsEpi<V>{yu, xhat, slack, Dc, 1.0 / beta, beta, 1.0 / gamma, gamma, c, xanc, xu, su,
-                              refine_active ? xstar : nullptr, idp, idd, bnd_w, lbv, ubv},
-                red);
+      const KktColsEpi<V> cols{yu, xhat, slack, Dc, 1.0 / beta, beta, 1.0 / gamma, gamma, c, xanc, xu, su,
+                               refine_active ? xstar : nullptr, idp, idd, bnd_w, lbv, ubv};
+      rows_pass<BT, 4>(tptr, tidx, torig, d.lgt, tblk, st,
+                       GlobalGather<KktColsEpi<V>>{cols, as_global((const double*)yu)}, red);
       wg_sum<4>(red, lds);
       const double dp = red[3];  // ||x0 - xhat||^2
       l2p        = sqrt(rp2);
@@ -1005,14 +1052,16 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
             tau                 = eta / omega;
             sigma               = eta * omega;
             rdp = sdp, rdd = sdd;
-            for (int j = tid; j < n; j += kBT) xstar[j] = fmin(fmax(xu[j], lbv[j]), ubv[j]);
-            for (int i = tid; i < m; i += kBT) ystar[i] = yu[i];
+            for (int j = tid; j < n; j += BT) xstar[j] = fmin(fmax(xu[j], lbv[j]), ubv[j]);
+            for (int i = tid; i < m; i += BT) ystar[i] = yu[i];
             __syncthreads();
             double rr[kMaxRed];
-            rows_pass(aptr, aidx, aorig, d.lga, ablk, st, BPlainEpi{xstar, ax64}, rr);
-            rows_pass(tptr, tidx, torig, d.lgt, tblk, st, BPlainEpi{ystar, aty64}, rr);
+            rows_pass<BT, 0>(aptr, aidx, aorig, d.lga, ablk, st,
+                             GlobalGather<BSpmvEpi<double*>>{{ax64}, as_global((const double*)xstar)}, rr);
+            rows_pass<BT, 0>(tptr, tidx, torig, d.lgt, tblk, st,
+                             GlobalGather<BSpmvEpi<double*>>{{aty64}, as_global((const double*)ystar)}, rr);
             __syncthreads();
-            for (int j = tid; j < n; j += kBT) {
+            for (int j = tid; j < n; j += BT) {
               const double dc = Dc[j], x = xstar[j];
               c_w[j]          = (V)((sdd * (c[j] - aty64[j])) * dc);
               V2 bb;
@@ -1024,7 +1073,7 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
               xanc[j]    = V(0);
               slack[j]   = V(0);
             }
-            for (int i = tid; i < m; i += kBT) {
+            for (int i = tid; i < m; i += BT) {
               const double r = Dr[i];
               V2 bb;
               bb.x       = (V)((sdp * (lc[i] - ax64[i])) * r);
@@ -1041,12 +1090,12 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
             refine_active = true;
             ++recentrings;
           } else {
-            for (int j = tid; j < n; j += kBT) {
+            for (int j = tid; j < n; j += BT) {
               const V v  = xhat[j];
               xanc[j]    = v;
               xs[cur][j] = v;
             }
-            for (int i = tid; i < m; i += kBT) {
+            for (int i = tid; i < m; i += BT) {
               const V v  = yhat[i];
               yanc[i]    = v;
               ys[cur][i] = v;
@@ -1076,17 +1125,19 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
         zero_red(red);
 #define CUOPT_BPRIMAL(MAJ, FP)                                                                              \
   do {                                                                                                        \
-    const PrimalStepEpi<V, MAJ, FP> e{ys[ci], xs[ci], c_w, bnd_w, xanc, xbar, xs[nx], xhat, slack, aty, &sc, jj,   \
-                                      refine_active};                                                         \
-    if (vec_in_lds) rows_pass(tptr, tidx, tw, d.lgt, tblk, st, LdsGather<decltype(e)>{e, as_lds(ys[ci])}, red);  \
-    else rows_pass(tptr, tidx, tw, d.lgt, tblk, st, GlobalGather<decltype(e)>{e, as_global(ys[ci])}, red);        \
+    PrimalStepEpi<V, MAJ, FP, true> e{ys[ci], xs[ci], c_w, bnd_w, xanc, xbar, xs[nx], xhat, slack, aty, &sc, jj,         \
+                                refine_active};                                                               \
+    e.begin();                                                                                               \
+    if (vec_in_lds) rows_pass<BT, 0>(tptr, tidx, tw, d.lgt, tblk, st, LdsGather<decltype(e)>{e, as_lds(ys[ci])}, red);  \
+    else rows_pass<BT, 0>(tptr, tidx, tw, d.lgt, tblk, st, GlobalGather<decltype(e)>{e, as_global(ys[ci])}, red);        \
   } while (0)
 #define CUOPT_BDUAL(MAJ, FP)                                                                                 \
   do {                                                                                                        \
-    const DualStepEpi<V, MAJ, FP> e{xbar, ys[ci], cb_w, yanc, ys[nx], yhat, ybar, &sc, jj,                         \
-                                    refine_active ? (const V*)kink : nullptr};                                  \
-    if (vec_in_lds) rows_pass(aptr, aidx, aw, d.lga, ablk, st, LdsGather<decltype(e)>{e, as_lds((const V*)xbar)}, red); \
-    else rows_pass(aptr, aidx, aw, d.lga, ablk, st, GlobalGather<decltype(e)>{e, as_global((const V*)xbar)}, red); \
+    DualStepEpi<V, MAJ, FP, true> e{xbar, ys[ci], cb_w, yanc, ys[nx], yhat, ybar, &sc, jj,                               \
+                              refine_active ? (const V*)kink : nullptr};                                        \
+    e.begin();                                                                                               \
+    if (vec_in_lds) rows_pass<BT, (FP) ? 1 : 0>(aptr, aidx, aw, d.lga, ablk, st, LdsGather<decltype(e)>{e, as_lds((const V*)xbar)}, red); \
+    else rows_pass<BT, (FP) ? 1 : 0>(aptr, aidx, aw, d.lga, ablk, st, GlobalGather<decltype(e)>{e, as_global((const V*)xbar)}, red); \
   } while (0)
         if (should_major) {
           if (fpe_step) CUOPT_BPRIMAL(true, true);
@@ -1109,7 +1160,8 @@ __global__ __launch_bounds__(kBT, kWgPerCu) void batch_pdlp_kernel(BatchArgs<V> 
           wg_sum<1>(red, lds);
           const double ny = red[0];
           zero_red(red);
-          rows_pass(tptr, tidx, tw, d.lgt, tblk, st, FpeEpi<V>{ybar, aty, xbar, xs[ci]}, red);
+          rows_pass<BT, 2>(tptr, tidx, tw, d.lgt, tblk, st,
+                           GlobalGather<FpeEpi<V>>{FpeEpi<V>{ybar, aty, xbar, xs[ci]}, as_global((const V*)ybar)}, red);
           wg_sum<2>(red, lds);
           if (post_restart) {
             fpe0_t[0] = ny;
@@ -1179,6 +1231,29 @@ void host_parallel_for(int count, F f)
   work(0);
   for (auto& x : th) x.join();
   if (err) std::rethrow_exception(err);
+}
+
+// Whether LPs of at least kWideNnz nonzeros get wide workgroups.  The launch takes at
+// least as long as its longest LP, and as the CU time of all of them over the CUs;
+// both are estimated per iteration (the LPs' iteration counts are not known) from
+// the measured 6 + 2.6 z us of a narrow workgroup (half a CU) and 6.5 + 1.3 z us of a
+// wide one, z being the LP's nonzeros in thousands.
+bool prefer_wide(const std::vector<BatchDesc>& desc, const std::vector<int>& active)
+{
+  int dev = 0, cus = 0;
+  CUOPT_HIP_CHECK(hipGetDevice(&dev));
+  CUOPT_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  double sum_n = 0.0, max_n = 0.0, sum_w = 0.0, max_w = 0.0;
+  for (int a : active) {
+    const double z  = 1e-3 * desc[a].nnz;
+    const bool w    = desc[a].nnz >= kWideNnz;
+    const double tn = 6.0 + 2.6 * z, tw = w ? 6.5 + 1.3 * z : tn;
+    sum_n += tn / wg_per_cu(kRef);
+    sum_w += tw / (w ? wg_per_cu(kWide) : wg_per_cu(kRef));
+    max_n = std::max(max_n, tn);
+    max_w = std::max(max_w, tw);
+  }
+  return std::max(sum_w / cus, max_w) < std::max(sum_n / cus, max_n);
 }
 
 template <typename V>
@@ -1253,18 +1328,25 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
       std::copy(ucs[a].begin(), ucs[a].end(), h_uc.get() + d.row0);
     }
   };
+  const bool wide = prefer_wide(desc, active);
   // row blocks of A and A^T for each LP
-  std::vector<std::vector<int>> ablocks(lps.size()), tblocks(lps.size());
+  std::vector<std::vector<int>> ablocks(lps.size()), tblocks(lps.size()), aref(lps.size()), tref(lps.size());
   {
     auto plan = [&](int t, int nt) {
       std::vector<int> cnt;
       for (int q = t; q < nb; q += nt) {
         const int a      = active[q];
         const LpHost& lp = *lps[a];
-        plan_row_blocks(lp.m, desc[a].lga, [&](int r) { return lp.rowptr[r + 1] - lp.rowptr[r]; }, ablocks[a]);
+        const auto alen  = [&](int r) { return lp.rowptr[r + 1] - lp.rowptr[r]; };
+        const auto tlen  = [&](int j) { return cnt[j]; };
         cnt.assign(lp.n, 0);
         for (int k = 0; k < desc[a].nnz; ++k) ++cnt[lp.colidx[k]];
-        plan_row_blocks(lp.n, desc[a].lgt, [&](int j) { return cnt[j]; }, tblocks[a]);
+        plan_row_blocks(lp.m, desc[a].lga, kRef, alen, aref[a]);
+        plan_row_blocks(lp.n, desc[a].lgt, kRef, tlen, tref[a]);
+        if (wide && desc[a].nnz >= kWideNnz) {
+          plan_row_blocks(lp.m, desc[a].lga, kWide, alen, ablocks[a]);
+          plan_row_blocks(lp.n, desc[a].lgt, kWide, tlen, tblocks[a]);
+        }
       }
     };
     const int nt = std::max(1, std::min<int>(16, (int)std::thread::hardware_concurrency()));
@@ -1275,17 +1357,26 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
   std::vector<int> h_blk;
   for (int a : active) {
     BatchDesc& d = desc[a];
-    d.ablk0      = (int)h_blk.size();
-    d.nablk      = (int)ablocks[a].size() - 1;
-    h_blk.insert(h_blk.end(), ablocks[a].begin(), ablocks[a].end());
-    d.tblk0 = (int)h_blk.size();
-    d.ntblk = (int)tblocks[a].size() - 1;
-    h_blk.insert(h_blk.end(), tblocks[a].begin(), tblocks[a].end());
+    auto put     = [&](const std::vector<int>& v, int& first, int& count) {
+      first = (int)h_blk.size();
+      count = (int)v.size() - 1;
+      h_blk.insert(h_blk.end(), v.begin(), v.end());
+    };
+    put(aref[a], d.aref0, d.naref);
+    put(tref[a], d.tref0, d.ntref);
+    d.ablk0 = d.aref0, d.nablk = d.naref;
+    d.tblk0 = d.tref0, d.ntblk = d.ntref;
+    if (wide && d.nnz >= kWideNnz) {
+      put(ablocks[a], d.ablk0, d.nablk);
+      put(tblocks[a], d.tblk0, d.ntblk);
+    }
   }
 
   // processing order: largest first
   std::vector<int> order(active);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return desc[x].nnz > desc[y].nnz; });
+  int nwide = 0;  // the first ones, by their order
+  while (wide && nwide < nb && desc[order[nwide]].nnz >= kWideNnz) ++nwide;
   std::vector<double> z0(std::max(max_m, 1));
   {
     std::mt19937 gen(1);
@@ -1297,8 +1388,12 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
   CUOPT_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   struct StreamGuard {
     hipStream_t s;
-    ~StreamGuard() { (void)hipStreamDestroy(s); }
-  } guard{s};
+    ~StreamGuard()
+    {
+      if (s) (void)hipStreamDestroy(s);
+    }
+  } guard{s}, beside{nullptr};
+  if (nwide > 0 && nwide < nb) CUOPT_HIP_CHECK(hipStreamCreateWithFlags(&beside.s, hipStreamNonBlocking));
   const size_t M = std::max(tot_m, 1), N = std::max(tot_n, 1), Z = std::max<long long>(tot_nnz, 1);
   DevArena arena;  // every working array below: one allocation
   auto d_desc = arena.take<BatchDesc>(std::max<size_t>(desc.size(), 1));
@@ -1358,6 +1453,7 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
   auto ax64 = arena.take<double>(refine ? M : 1);
   auto aty64 = arena.take<double>(refine ? N : 1);
   auto kink = arena.take<V>(refine ? M : 1);
+  auto red_rows = arena.take<double>(nwide > 0 ? 4 * (M + N) : 1);
   auto out = arena.take<BatchOut>(std::max<size_t>(lps.size(), 1));
   auto lz = arena.take<double>(std::is_same<V, float>::value ? std::max<size_t>(lps.size(), 1) * kLzStride : 1);
   arena.commit();
@@ -1483,6 +1579,7 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
   args.z0 = dz0.get();
   args.out = out.get();
   args.lz  = lz.get();
+  args.red_rows = red_rows.get();
   args.tol_ap = st.abs_primal;
   args.tol_rp = st.rel_primal;
   args.tol_ad = st.abs_dual;
@@ -1504,35 +1601,53 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
     const double ticks = std::max(1.0, st.time_limit * 1e3 * (double)khz);
     args.tick_limit    = ticks >= 1.8e19 ? 0ULL : (unsigned long long)ticks;
   }
-  {
-    // LDS: the row-block stage and, at the end, each LP's gathered vectors when
-    // they fit; as much as the per-workgroup limit and a CU's LDS divided by
-    // kWgPerCu allow.
+  // LDS of a width: the row-block stage and, at the end, each LP's gathered vectors
+  // when they fit; as much as the per-workgroup limit and a CU's LDS divided by the
+  // workgroups that it holds (their register budget) allow.
+  auto lds_of = [](int bt) {
     int dev = 0, per_block = 0, per_cu = 0;
     CUOPT_HIP_CHECK(hipGetDevice(&dev));
     CUOPT_HIP_CHECK(hipDeviceGetAttribute(&per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     CUOPT_HIP_CHECK(hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev));
-    const long long static_lds = 4096;  // the kernel's own __shared__ arrays, rounded up
-    long long cap = std::min<long long>(per_block, per_cu / kWgPerCu) - static_lds;
-    if (cap < kStageBytes) throw std::runtime_error("batch solve: the device has too little LDS per workgroup");
-    args.lds_bytes = (int)cap;  // two workgroups per CU either way (their register budget)
-  }
+    // the kernel's own __shared__ arrays (4 bytes a lane and about 400), rounded up
+    const long long static_lds = 3072 + 4 * bt;
+    const long long cap        = std::min<long long>(per_block, per_cu / wg_per_cu(bt)) - static_lds;
+    if (cap < stage_bytes(bt)) throw std::runtime_error("batch solve: the device has too little LDS per workgroup");
+    return (int)cap;
+  };
   // HIP events around the persistent launch: its device time is the batch's loop time.
-  hipEvent_t ev[2] = {nullptr, nullptr};
+  hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   struct EventGuard {
     hipEvent_t* e;
     ~EventGuard()
     {
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 3; ++i)
         if (e[i]) (void)hipEventDestroy(e[i]);
     }
   } ev_guard{ev};
   CUOPT_HIP_CHECK(hipEventCreate(&ev[0]));
   CUOPT_HIP_CHECK(hipEventCreate(&ev[1]));
+  CUOPT_HIP_CHECK(hipEventCreateWithFlags(&ev[2], hipEventDisableTiming));
   CUOPT_HIP_CHECK(hipEventRecord(ev[0], s));
-  if (nb > 0) {
-    hipLaunchKernelGGL(batch_pdlp_kernel<V>, dim3(nb), dim3(kBT), (unsigned)args.lds_bytes, s, args);
+  // The wide LPs first; with both widths the narrow ones run beside them on a stream
+  // of their own, between two events of this one.
+  const int nnarrow = nb - nwide;
+  hipStream_t s2    = nwide > 0 && nnarrow > 0 ? beside.s : s;
+  if (s2 != s) CUOPT_HIP_CHECK(hipStreamWaitEvent(s2, ev[0], 0));
+  if (nwide > 0) {
+    args.lds_bytes = lds_of(kWide);
+    hipLaunchKernelGGL((batch_pdlp_kernel<V, kWide>), dim3(nwide), dim3(kWide), (unsigned)args.lds_bytes, s, args);
     CUOPT_HIP_CHECK(hipGetLastError());
+  }
+  if (nnarrow > 0) {
+    args.order     = d_order.get() + nwide;
+    args.lds_bytes = lds_of(kRef);
+    hipLaunchKernelGGL((batch_pdlp_kernel<V, kRef>), dim3(nnarrow), dim3(kRef), (unsigned)args.lds_bytes, s2, args);
+    CUOPT_HIP_CHECK(hipGetLastError());
+  }
+  if (s2 != s) {
+    CUOPT_HIP_CHECK(hipEventRecord(ev[2], s2));
+    CUOPT_HIP_CHECK(hipStreamWaitEvent(s, ev[2], 0));
   }
   CUOPT_HIP_CHECK(hipEventRecord(ev[1], s));
   // Host work while the launch runs: release the input staging once its uploads

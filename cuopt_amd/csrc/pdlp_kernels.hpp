@@ -92,8 +92,27 @@ __device__ inline V halpern_weight(const StepScalars* sc, int j)
   return (V)((double)(kr + 1) / (double)(kr + 2));
 }
 
+// v holds the same value in every lane: say so to the compiler, which then keeps it (and
+// what is computed from it: a batch's restart and termination scalars) in scalar
+// registers instead of one vector register or pair per value.
+__device__ inline float uniform_value(float v)
+{
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+__device__ inline double uniform_value(double v)
+{
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b & 0xffffffffu));
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // ---- primal step over rows of A~^T (columns j): AtY, projection, reflection, Halpern.
-template <typename V, bool MAJOR, bool FPE>
+// HOIST (the batch kernel, many rows per lane): begin() sets the step's scalars once
+// per pass; without it each row evaluates them, which the tiled kernels overlap with
+// their memory accesses (evaluated before their first loads, they took the steps of
+// the 500 k x 1 M LP about 1 % longer).
+template <typename V, bool MAJOR, bool FPE, bool HOIST = false>
 struct PrimalStepEpi {
   using Mat = V;
   using Acc = typename AccFor<V>::type;
@@ -114,6 +133,12 @@ struct PrimalStepEpi {
   // Recentred (refined) solves: store only the part (x-hat - x) / tau of the slack; the
   // termination check adds the FP64 reduced cost of the corrected point.
   bool small_slack;
+  V htau = V(0), hw = V(0);
+  __device__ void begin()
+  {
+    htau = uniform_value((V)sc->tau);
+    hw   = uniform_value(halpern_weight<V>(sc, j));
+  }
   __device__ bool skip() const { return false; }
   struct Pre {
     V x, c, x0;
@@ -123,8 +148,8 @@ struct PrimalStepEpi {
   __device__ Pre load(int r) const { return Pre{x[r], c[r], x0[r], bnd[r]}; }
   __device__ void row(int r, const Acc& aty, const Pre& p, double (&)[kMaxRed]) const
   {
-    const V tau     = (V)sc->tau;
-    const V w       = halpern_weight<V>(sc, j);
+    const V tau     = HOIST ? htau : (V)sc->tau;
+    const V w       = HOIST ? hw : halpern_weight<V>(sc, j);
     const V next    = p.x - tau * aty.rsub(p.c);
     const V clamped = mx(mn(next, p.b.y), p.b.x);
     const V xb      = V(2) * clamped - p.x;
@@ -176,7 +201,7 @@ struct TilePipelining<PrimalStepEpi<double, MAJOR, FPE>, TILE> {
 };
 
 // ---- dual step over rows of A~ (rows i): A x-bar, projection, reflection, Halpern.
-template <typename V, bool MAJOR, bool FPE>
+template <typename V, bool MAJOR, bool FPE, bool HOIST = false>
 struct DualStepEpi {
   using Mat = V;
   using Acc = typename AccFor<V>::type;
@@ -195,6 +220,12 @@ struct DualStepEpi {
   // dual objective term, which sits at y = 0 in the original problem and at
   // -Dd * y* / Dr in the coordinates of a correction problem.
   const V* kink;
+  V hsigma = V(0), hw = V(0);  // HOIST: set by begin(), as in the primal step
+  __device__ void begin()
+  {
+    hsigma = uniform_value((V)sc->sigma);
+    hw     = uniform_value(halpern_weight<V>(sc, j));
+  }
   __device__ bool skip() const { return false; }
   struct Pre {
     V y, y0, k;
@@ -204,8 +235,8 @@ struct DualStepEpi {
   __device__ Pre load(int r) const { return Pre{y[r], y0[r], kink ? kink[r] : V(0), cb[r]}; }
   __device__ void row(int r, const Acc& ax, const Pre& p, double (&red)[kMaxRed]) const
   {
-    const V sigma = (V)sc->sigma;
-    const V w     = halpern_weight<V>(sc, j);
+    const V sigma = HOIST ? hsigma : (V)sc->sigma;
+    const V w     = HOIST ? hw : halpern_weight<V>(sc, j);
     V nd;
     if (kink) {
       // The projection of the original problem moved to the kink k, written as

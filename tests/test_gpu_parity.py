@@ -10,6 +10,7 @@ Tolerances, stated per test:
 * FP32-mixed solve at tol: objective within 10 tol of the closed-form optimum
 """
 
+import dataclasses
 import json
 import os
 
@@ -845,3 +846,28 @@ def test_reference_parser_fixtures_solve_to_the_highs_optimum(fname):
         assert abs(r.primal_objective - obj) <= 1e-6 * (1 + abs(obj)), (fname, precision)
         if precision == "fp64":
             assert r.iterations == O.solve(lp, tol=1e-8)["iterations"], fname
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_batch_result_does_not_depend_on_the_workgroup_width(prec):
+    # A few LPs get wide workgroups; the same LPs among thousands get narrow ones.  Every
+    # reduction keeps one order, so an LP's result is the same bit for bit.  Sizes around
+    # the smallest wide LP (2 000 nonzeros) and past a block's rows, with a row longer
+    # than a staged block (2 552 nonzeros).
+    import scipy.sparse as sp
+
+    few = [G.random_lp(m=m, n=int(2.5 * m), seed=m) for m in (97, 101, 103, 257, 1300, 1803)]
+    lp = G.random_lp(m=60, n=3001, seed=5)
+    dense = sp.vstack([lp.to_scipy(), sp.csr_matrix(np.linspace(0.5, 1.5, lp.n)[None, :])]).tocsr()
+    b = np.append(lp.con_lb, (dense @ lp.x_opt)[-1])
+    few.append(dataclasses.replace(lp, m=lp.m + 1, row_offsets=dense.indptr.astype(np.int32),
+                                   col_indices=dense.indices.astype(np.int32), values=dense.data, con_lb=b, con_ub=b))
+    many = few + [G.random_lp(m=101 + i % 7, n=250, seed=i) for i in range(6000)]
+    kw = dict(tol=1e-6, precision=prec, iteration_limit=600, time_limit=60.0)
+    alone, among = c_api.batch_solve(few, **kw), c_api.batch_solve(many, **kw)
+    for i, (p, q) in enumerate(zip(alone, among)):
+        assert (p.status, p.iterations) == (q.status, q.iterations), i
+        for f in ("x", "y", "reduced_cost"):
+            assert np.array_equal(getattr(p, f), getattr(q, f)), (i, f)
+        for k in ("eta0", "omega", "power_iterations", "l2_primal_residual", "l2_dual_residual", "gap"):
+            assert p.info[k] == q.info[k], (i, k)
