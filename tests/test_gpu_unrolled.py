@@ -291,3 +291,37 @@ def test_full_size_fp64_vjp_matches_central_differences():
             # measured (c): 1.7e-3, 1.4e-4, 6.7e-6 at h = 1e-6, 1e-7, 1e-8; rounding takes over at 1e-9
             assert min(errs.values()) <= 2e-5, errs
             assert errs[1e-8] < errs[1e-7] < errs[1e-6], errs
+
+
+@pytest.mark.parametrize("per_member_bounds", [False, True])
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_member_result_does_not_depend_on_the_slab_shape(monkeypatch, prec, per_member_bounds):
+    # Batch sizes around the slab widths (4, 8, 16, 32) in every shape of the SpMM kernels
+    # (10 x lanes per row + members per lane), on a ragged matrix: a member's point and
+    # gradients are those it has in a batch of its own, bit for bit (each is the sum of
+    # the same terms in the same order whatever the shape).
+    lp, _ = ragged_lp(seed=4, m=1100, n=1500)
+    op = UnrolledPDHG(lp, ridge=1e-3, steps=24, checkpoint_every=7, precision=prec)
+    rng = np.random.default_rng(9)
+    top = 33
+    c = lp.c[None, :] + 0.1 * rng.normal(size=(top, lp.n))
+    slack = rng.uniform(0.1, 0.5, size=(top, lp.m))
+    gx, gy = rng.normal(size=(top, lp.n)), rng.normal(size=(top, lp.m))
+
+    def run(members):
+        lc = lp.con_lb - slack[members] if per_member_bounds else lp.con_lb
+        uc = lp.con_ub + slack[members] if per_member_bounds else lp.con_ub
+        ct, lt, ut = (torch.tensor(v, device=DEV, requires_grad=True) for v in (c[members], lc, uc))
+        x, y = op(ct, lt, ut)
+        torch.autograd.backward([x, y], [torch.tensor(gx[members], device=DEV), torch.tensor(gy[members], device=DEV)])
+        grads = [ct.grad] + ([lt.grad, ut.grad] if per_member_bounds else [])
+        return [v.detach().cpu().numpy() for v in (x, y, *grads)]
+
+    alone = [run([i]) for i in range(top)]
+    for shape in (None, 41, 81, 82, 84, 161):
+        if shape:
+            monkeypatch.setenv("CUOPT_AMD_UNR_SHAPE", str(shape))
+        for B in (2, 4, 5, 8, 9, 16, 17, 33):
+            for k, v in enumerate(run(list(range(B)))):
+                for i in range(B):
+                    assert np.array_equal(v[i], alone[i][k][0]), (shape, B, k, i)
