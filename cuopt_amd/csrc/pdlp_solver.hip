@@ -34,6 +34,7 @@
 #include "common.hpp"
 #include "lp_types.hpp"
 #include "pdlp_kernels.hpp"
+#include "small_block.hpp"
 #include "tile_plan.hpp"
 
 namespace cuopt_amd {
@@ -1150,6 +1151,8 @@ class PdlpSolver {
     if (stream_) (void)hipStreamDestroy(stream_);
     if (h_scal_) (void)hipHostFree(h_scal_);
     if (h_step_) (void)hipHostFree(h_step_);
+    if (h_power_) (void)hipHostFree(h_power_);
+    if (h_checks_) (void)hipHostFree(h_checks_);
   }
 
   SolveResult run();
@@ -1175,7 +1178,13 @@ class PdlpSolver {
     *h_step_ = StepScalars{tau_, sigma_, kr_, 0};
     CUOPT_HIP_CHECK(hipMemcpyAsync(step_sc_.get(), h_step_, sizeof(StepScalars), hipMemcpyHostToDevice, stream_));
   }
-  void evaluate_kkt();
+  void evaluate_kkt(const Tolerances& tol);
+  void take_kkt();
+  KktPointF<V> kkt_point() const;
+  KktRowsEpi<V> kkt_rows() const;
+  KktColsEpi<V> kkt_cols() const;
+  int small_rounds(size_t lds_bytes) const;
+  void launch_small(long long k, int count, long long limit, bool restarted, const Tolerances& tol);
   void launch_step(int j, bool major, bool fpe, double* ny_slot, double* fpe_slot);
   void finish(SolveResult& R, int status);
   int pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine);
@@ -1210,6 +1219,7 @@ class PdlpSolver {
   hipStream_t stream_ = nullptr;
   double* h_scal_     = nullptr;
   StepScalars* h_step_ = nullptr;
+  PowerState* h_power_ = nullptr;
 
   MatStruct A_, AT_;
   DevBuf<double> a_orig_, at_orig_, a_s_, at_s_;
@@ -1271,6 +1281,9 @@ class PdlpSolver {
   int cur_ = 0;
   hipEvent_t* ev_ = nullptr;  // events of the current timed iteration (benchmark window)
   bool use_graphs_ = true;
+  int small_       = 0;      // rounds of the one-workgroup blocks (small_block.hpp); 0: tiled launches
+  double* h_checks_ = nullptr;  // their records, one per check, and the number of checks
+  int checks_made_ = 0, checks_read_ = 0;
   std::map<std::string, hipGraphExec_t> graphs_;  // captured iteration blocks by pattern
 
   // recentring: the FP64 point (x*, y*), A x*, A^T y*, dual kinks
@@ -1614,6 +1627,23 @@ void PdlpSolver<V>::power_iteration()
   PowerState h{};
   h.nrm = std::sqrt(h_scal_[S_SETUP0]);
   CUOPT_HIP_CHECK(hipMemcpyAsync(st.get(), &h, sizeof(h), hipMemcpyHostToDevice, stream_));
+  if (const int rounds = small_rounds(small_power_lds_bytes(m_, n_))) {
+    if (!h_power_) CUOPT_HIP_CHECK(hipHostMalloc((void**)&h_power_, sizeof(PowerState), hipHostMallocDefault));
+    const SmallPowerArgs args{m_, n_, A_.ptr.get(), A_.idx.get(), AT_.ptr.get(), AT_.idx.get(), A_.plan.tiles.get(),
+                              AT_.plan.tiles.get(), A_.plan.meta.get(), AT_.plan.meta.get(), A_.plan.ntiles,
+                              AT_.plan.ntiles, a_s_.get(), at_s_.get(), za.get(), h.nrm, 1e-4, 5000, h_power_};
+    const unsigned lds = (unsigned)small_power_lds_bytes(m_, n_);
+    if (rounds == 1)
+      hipLaunchKernelGGL(small_power_kernel<1>, dim3(1), dim3(kSmallThreads), lds, stream_, args);
+    else
+      hipLaunchKernelGGL(small_power_kernel<kSmallRounds>, dim3(1), dim3(kSmallThreads), lds, stream_, args);
+    CUOPT_HIP_CHECK(hipGetLastError());
+    CUOPT_HIP_CHECK(hipStreamSynchronize(stream_));
+    sigma_max_sq_ = h_power_->s2;
+    power_iters_  = (int)h_power_->iters;
+    eta_          = 0.998 / std::sqrt(sigma_max_sq_);
+    return;
+  }
   double* zo = za.get();
   double* zn = zb.get();
   auto launch_batch = [&](int batch) {
@@ -1719,28 +1749,94 @@ void PdlpSolver<V>::init_iterates()
 }
 
 template <typename V>
-void PdlpSolver<V>::evaluate_kkt()
+KktPointF<V> PdlpSolver<V>::kkt_point() const
 {
-  const double ib = 1.0 / beta_, ig = 1.0 / gamma_;
-  const bool rf   = refine_active_;
-  const double* xs = rf ? xstar_.get() : nullptr;
-  const double* ys = rf ? ystar_.get() : nullptr;
-  const double idp = rf ? 1.0 / refine_.dp : 1.0, idd = rf ? 1.0 / refine_.dd : 1.0;
+  return KktPointF<V>{xhat_.get(), Dc_.get(), 1.0 / beta_, refine_active_ ? xstar_.get() : nullptr,
+                      refine_active_ ? 1.0 / refine_.dp : 1.0, xu_.get()};
+}
+
+template <typename V>
+KktRowsEpi<V> PdlpSolver<V>::kkt_rows() const
+{
+  const bool rf = refine_active_;
+  return KktRowsEpi<V>{xu_.get(), yhat_.get(), Dr_.get(), 1.0 / gamma_, gamma_, cb_orig_.get(), y0_.get(), yu_.get(),
+                       rf ? xstar_.get() : nullptr, rf ? ystar_.get() : nullptr, rf ? 1.0 / refine_.dp : 1.0,
+                       rf ? 1.0 / refine_.dd : 1.0, st_.per_constraint_residual ? rp_res_.get() : nullptr};
+}
+
+template <typename V>
+KktColsEpi<V> PdlpSolver<V>::kkt_cols() const
+{
+  const bool rf = refine_active_;
+  return KktColsEpi<V>{yu_.get(), xhat_.get(), slack_.get(), Dc_.get(), 1.0 / beta_, beta_, 1.0 / gamma_, gamma_,
+                       c_orig_.get(), x0_.get(), xu_.get(), su_.get(), rf ? xstar_.get() : nullptr,
+                       rf ? 1.0 / refine_.dp : 1.0, rf ? 1.0 / refine_.dd : 1.0, bnd_w_.get(), lb_orig_.get(),
+                       ub_orig_.get(), st_.per_constraint_residual ? rd_res_.get() : nullptr};
+}
+
+// Rounds of the one-workgroup kernels (small_block.hpp) when the LP's tiles and vectors
+// fit them, else 0.  CUOPT_AMD_SMALL=0 turns them off, for comparisons.
+template <typename V>
+int PdlpSolver<V>::small_rounds(size_t lds_bytes) const
+{
+  if (const char* e = std::getenv("CUOPT_AMD_SMALL"))
+    if (std::atoi(e) == 0) return 0;
+  if (st_.bench_steps > 0 || st_.per_constraint_residual) return 0;
+  if (A_.plan.nlong > 0 || AT_.plan.nlong > 0 || A_.tile > kSmallTile || AT_.tile > kSmallTile) return 0;
+  const int tiles = std::max(A_.plan.ntiles, AT_.plan.ntiles);
+  if (tiles > kSmallTiles) return 0;
+  int dev = 0, per_block = 0;
+  CUOPT_HIP_CHECK(hipGetDevice(&dev));
+  CUOPT_HIP_CHECK(hipDeviceGetAttribute(&per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  if (lds_bytes + 4096 > (size_t)per_block) return 0;  // beside the kernels' own arrays (under 3 KB)
+  return tiles <= kSmallGroups ? 1 : kSmallRounds;
+}
+
+// Up to `count` iterations from k with the termination checks on the way and the one
+// after them, in one launch, which ends at the first check that meets `tol` or lies
+// `limit` iterations on.
+template <typename V>
+void PdlpSolver<V>::launch_small(long long k, int count, long long limit, bool restarted, const Tolerances& tol)
+{
+  const int c = cur_;
+  const SmallArgs<V> args{m_, n_, A_.ptr.get(), A_.idx.get(), AT_.ptr.get(), AT_.idx.get(), A_.plan.tiles.get(),
+                          AT_.plan.tiles.get(), A_.plan.meta.get(), AT_.plan.meta.get(), A_.plan.ntiles,
+                          AT_.plan.ntiles, a_w_.get(), at_w_.get(), a_orig_.get(), at_orig_.get(), x_[c].get(),
+                          y_[c].get(), x_[c ^ 1].get(), x0_.get(), y0_.get(), c_w_.get(), bnd_w_.get(), cb_w_.get(),
+                          refine_active_ ? kink_.get() : nullptr, xhat_.get(), yhat_.get(), slack_.get(), aty_.get(),
+                          ybar_.get(), StepScalars{tau_, sigma_, kr_, 0}, refine_active_, k, count,
+                          (int)std::min<long long>(limit, count), restarted, tol.ap + tol.rp * b_norm_,
+                          tol.ad + tol.rd * c_norm_, tol.ag, tol.rg, obj_sf_, obj_off_, kkt_point(), kkt_rows(),
+                          kkt_cols(), h_checks_, S_COUNT, S_KKT_RP2, S_KKT_RD2, S_FPE_NY, S_FPE0_NY,
+                          reinterpret_cast<int*>(h_checks_ + kSmallChecks * S_COUNT)};
+  const unsigned lds = (unsigned)small_lds_bytes<V>(m_, n_);
+  if (small_ == 1)
+    hipLaunchKernelGGL((small_block_kernel<V, 1>), dim3(1), dim3(kSmallThreads), lds, stream_, args);
+  else
+    hipLaunchKernelGGL((small_block_kernel<V, kSmallRounds>), dim3(1), dim3(kSmallThreads), lds, stream_, args);
+  CUOPT_HIP_CHECK(hipGetLastError());
+  CUOPT_HIP_CHECK(hipStreamSynchronize(stream_));
+  checks_made_ = *reinterpret_cast<const int*>(h_checks_ + kSmallChecks * S_COUNT);
+  checks_read_ = 0;
+}
+
+template <typename V>
+void PdlpSolver<V>::evaluate_kkt(const Tolerances& tol)
+{
+  if (small_) {  // the launch before has evaluated its checks; nothing has run before the first one
+    if (checks_read_ == checks_made_) launch_small(0, 0, 0, false, tol);
+    std::copy_n(h_checks_ + (size_t)checks_read_++ * S_COUNT, (size_t)S_COUNT, h_scal_);
+    take_kkt();
+    return;
+  }
   // xu_ holds the gathered point until the column pass writes the final x there.
-  launch_ew(n_, nullptr, KktPointF<V>{xhat_.get(), Dc_.get(), ib, xs, idp, xu_.get()}, stream_);
+  launch_ew(n_, nullptr, kkt_point(), stream_);
   const bool per = st_.per_constraint_residual;
   if (per && rp_res_.size() < (size_t)std::max(m_, 1)) rp_res_.resize(std::max(m_, 1));
   if (per && rd_res_.size() < (size_t)std::max(n_, 1)) rd_res_.resize(std::max(n_, 1));
-  launch_tiled(A_, a_orig_.get(), red_.get(),
-               KktRowsEpi<V>{xu_.get(), yhat_.get(), Dr_.get(), ig, gamma_, cb_orig_.get(), y0_.get(), yu_.get(), xs,
-                             ys, idp, idd, per ? rp_res_.get() : nullptr},
-               stream_);
+  launch_tiled(A_, a_orig_.get(), red_.get(), kkt_rows(), stream_);
   launch_reduce(red_.get(), A_.plan.red_blocks(), 3, scal_.get() + S_KKT_RP2, stream_);
-  launch_tiled(AT_, at_orig_.get(), red_.get(),
-               KktColsEpi<V>{yu_.get(), xhat_.get(), slack_.get(), Dc_.get(), ib, beta_, ig, gamma_, c_orig_.get(),
-                             x0_.get(), xu_.get(), su_.get(), xs, idp, idd, bnd_w_.get(), lb_orig_.get(),
-                             ub_orig_.get(), per ? rd_res_.get() : nullptr},
-               stream_);
+  launch_tiled(AT_, at_orig_.get(), red_.get(), kkt_cols(), stream_);
   launch_reduce(red_.get(), AT_.plan.red_blocks(), 4, scal_.get() + S_KKT_RD2, stream_);
   if (per) {
     const int ab = st_.per_constraint_absolute;
@@ -1752,6 +1848,14 @@ void PdlpSolver<V>::evaluate_kkt()
     CUOPT_HIP_CHECK(hipGetLastError());
   }
   read_scalars();
+  take_kkt();
+}
+
+// The residuals and objectives of the scalar record that was just read.
+template <typename V>
+void PdlpSolver<V>::take_kkt()
+{
+  const bool per  = st_.per_constraint_residual;
   const double* s = h_scal_;
   l2p_            = std::sqrt(s[S_KKT_RP2]);
   l2d_            = std::sqrt(s[S_KKT_RD2]);
@@ -1949,6 +2053,9 @@ SolveResult PdlpSolver<V>::run()
   tau_   = eta_ / omega_;
   sigma_ = eta_ * omega_;
   init_iterates();
+  small_ = small_rounds(small_lds_bytes<V>(m_, n_));
+  if (small_)
+    CUOPT_HIP_CHECK(hipHostMalloc((void**)&h_checks_, (kSmallChecks * S_COUNT + 1) * sizeof(double), hipHostMallocDefault));
   if constexpr (!std::is_same<V, double>::value) {
     CUOPT_HIP_CHECK(hipStreamSynchronize(stream_));
     a_s_.release();
@@ -2126,7 +2233,7 @@ int PdlpSolver<V>::pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine)
     if (bench && k >= bench_w && k < bench_end) ++bench_checks;
     // ---- termination check (k is a check iteration) ----
     const bool is_major = ((k % kMajor) == 0 && k > 0) || k <= 0;
-    evaluate_kkt();
+    evaluate_kkt(tol);
     ++checks_;
     if (restarted_prev) {
       fpe  = std::sqrt((h_scal_[S_FPE0_NX] * omega_ + h_scal_[S_FPE0_NY] / omega_) + 2.0 * h_scal_[S_FPE0_I] * eta_);
@@ -2146,7 +2253,8 @@ int PdlpSolver<V>::pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine)
     if (st_.stop_on_nan && (std::isnan(l2p_) || std::isnan(l2d_) || std::isnan(gap_)))
       return done(CUOPT_TERIMINATION_STATUS_NUMERICAL_ERROR);
     if (st_.save_best_primal_so_far && !bench) record_best(tol);  // pdlp.cu:1171-1175
-    if (elapsed() >= st_.time_limit) {
+    const bool ahead = small_ && checks_read_ < checks_made_;  // the point is that of a later check
+    if (!ahead && elapsed() >= st_.time_limit) {
       if (st_.save_best_primal_so_far && !bench) restore_best();  // pdlp.cu:341-347
       return done(CUOPT_TERIMINATION_STATUS_TIME_LIMIT);
     }
@@ -2212,15 +2320,14 @@ int PdlpSolver<V>::pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine)
     }
     R.trace[rec + 6] = restarted ? 1.0 : 0.0;
     R.trace[rec + 7] = omega_;
-    upload_step_scalars();
-
     // ---- PDHG iterations up to the next check ----
     long long next = k + 1;
     while (!is_check(next)) ++next;
     periodic_prev = false;
+    if (!small_) upload_step_scalars();
     const bool evented = bench && k >= bench_end;
     std::string key;
-    if (use_graphs_ && !evented) {
+    if (use_graphs_ && !evented && !small_) {
       key = std::to_string(next - k) + (restarted ? "R" : "") + (refine_active_ ? "K:" : ":");
       for (long long s = k; s < next; ++s) {
         const long long s2 = s + 2;
@@ -2251,7 +2358,17 @@ int PdlpSolver<V>::pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine)
     };
     for (long long s = k; s < next; ++s)
       if (((s + 1) % kMajor) == 0) periodic_prev = true;
-    if (!key.empty()) {
+    if (small_) {
+      // One launch runs up to the next restart test (every 200 iterations) and makes the
+      // checks on the way; their records are read one by one here, as if each had been
+      // waited for.  Options that may end the solve at a check for another reason than
+      // its optimality, or keep its point, get a launch per check.
+      if (checks_read_ == checks_made_) {
+        const bool each     = st_.first_primal_feasible || st_.stop_on_nan || st_.save_best_primal_so_far;
+        const long long end = each ? next : (k / kMajor + 1) * kMajor;
+        launch_small(k, (int)(end - k), st_.iteration_limit - (k0 + k), restarted, tol);
+      }
+    } else if (!key.empty()) {
       // Blocks have even length, so the ping-pong buffers are in the same state
       // at every block start and a captured block is valid for every replay.
       auto it = graphs_.find(key);

@@ -871,3 +871,51 @@ def test_batch_result_does_not_depend_on_the_workgroup_width(prec):
             assert np.array_equal(getattr(p, f), getattr(q, f)), (i, f)
         for k in ("eta0", "omega", "power_iterations", "l2_primal_residual", "l2_dual_residual", "gap"):
             assert p.info[k] == q.info[k], (i, k)
+
+
+def _ragged_small_lp(m, n, seed):
+    # Rows of 0 to 60 nonzeros, empty columns, inequality and equality rows.
+    import scipy.sparse as sp
+
+    rng = np.random.default_rng(seed)
+    rows = [rng.choice(n - 3, size=min(n - 3, 0 if i % 11 == 4 else 60 if i % 29 == 7 else int(rng.integers(1, 9))),
+                       replace=False) for i in range(m)]
+    ptr = np.cumsum([0] + [len(r) for r in rows])
+    idx = np.concatenate([np.sort(r) for r in rows])
+    A = sp.csr_matrix((rng.normal(size=len(idx)), idx, ptr), shape=(m, n))
+    x0, y0 = np.where(rng.random(n) < 0.5, rng.random(n), 0.0), rng.normal(size=m)
+    le = np.arange(m) % 3 == 1
+    y0[le] = 0.0
+    b = A @ x0
+    return G.LP(m=m, n=n, row_offsets=A.indptr.astype(np.int32), col_indices=A.indices.astype(np.int32), values=A.data,
+                c=A.T @ y0 + np.where(x0 == 0, rng.random(n), 0.0), con_lb=np.where(le, -np.inf, b),
+                con_ub=np.where(le, b + 0.5, b), var_lb=np.zeros(n), var_ub=np.full(n, 5.0))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+@pytest.mark.parametrize("lp", [G.random_lp(m=1, n=2, nnz_per_col=1, seed=1), G.random_lp(m=51, n=127, seed=2),
+                                G.random_lp(m=53, n=128, seed=3), G.random_lp(m=203, n=509, seed=4),
+                                G.random_lp(m=207, n=511, seed=5), G.random_lp(m=400, n=1019, seed=6),
+                                G.random_lp(m=409, n=1021, seed=7), _ragged_small_lp(1030, 700, 8),
+                                _ragged_small_lp(300, 1500, 9)], ids=lambda lp: f"{lp.m}x{lp.n}")
+def test_small_lp_in_one_workgroup_is_the_tiled_solve(monkeypatch, lp, prec):
+    # LPs of 1 to 8 tiles per matrix (and just past them) run in one workgroup; every sum
+    # keeps the order of the tiled kernels, so the solve is the same bit for bit: with
+    # restarts and refinement, at an iteration limit between checks, with an option
+    # that takes a launch per check, and from an initial point.
+    rng = np.random.default_rng(0)
+    start = dict(x_init=rng.random(lp.n), y_init=rng.normal(size=lp.m))
+    for kw in (dict(tol=1e-8, iteration_limit=1600), dict(tol=1e-4), dict(tol=0.0, iteration_limit=233),
+               dict(tol=1e-6, iteration_limit=450, params={"save_best_primal_so_far": 1}),
+               dict(tol=1e-5, iteration_limit=800, **start)):
+        kw.setdefault("iteration_limit", 3000)
+        got = []
+        for small in ("0", "1"):
+            monkeypatch.setenv("CUOPT_AMD_SMALL", small)
+            got.append(c_api.solve(lp, precision=prec, time_limit=60.0, **kw))
+        a, b = got
+        assert (a.status, a.iterations) == (b.status, b.iterations), kw
+        for f in ("x", "y", "reduced_cost", "trace"):
+            assert np.array_equal(getattr(a, f), getattr(b, f), equal_nan=True), (kw, f)
+        for k in ("eta0", "power_iterations", "omega", "restarts", "checks", "refine_rounds", "gap"):
+            assert a.info[k] == b.info[k], (kw, k)
