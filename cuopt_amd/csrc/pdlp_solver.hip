@@ -43,25 +43,44 @@ namespace cuopt_amd {
 // Generic kernels
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(1024) void reduce_partials_kernel(const double* __restrict__ part,
-                                                               int nblocks,
-                                                               int nred,
-                                                               double* __restrict__ out,
-                                                               const double* skip)
+// Sums of NR interleaved partials (part[b * NR + k]) into out, one workgroup.
+template <int NR>
+__device__ inline void reduce_partials(const double* __restrict__ part, int nblocks, double* __restrict__ out,
+                                       double (*lds)[1024])
 {
-  __shared__ double lds[1024];
-  if (skip && *skip != 0.0) return;
-  for (int k = 0; k < nred; ++k) {
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) s += part[(size_t)b * nred + k];
-    lds[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-      if ((int)threadIdx.x < off) lds[threadIdx.x] += lds[threadIdx.x + off];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[k] = lds[0];
-    __syncthreads();
+  const int tid = threadIdx.x;
+  double s[NR];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) s[k] = 0.0;
+  for (int b = tid; b < nblocks; b += 1024)
+#pragma unroll
+    for (int k = 0; k < NR; ++k) s[k] += part[(size_t)b * NR + k];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) lds[k][tid] = s[k];
+  __syncthreads();
+  if (tid < NR * kWave) {
+    const double v = tree_1024(lds[tid / kWave]);
+    if (tid % kWave == 0) out[tid / kWave] = v;
+  }
+}
+
+// One reduction, of nred partials per block.
+struct Reduction {
+  const double* part;
+  int nblocks, nred;
+  double* out;
+};
+
+// Two reductions at once, one workgroup each.
+__global__ __launch_bounds__(1024) void reduce_partials_kernel(Reduction a, Reduction b)
+{
+  __shared__ double lds[4][1024];
+  const Reduction r = blockIdx.x == 0 ? a : b;
+  switch (r.nred) {
+    case 1: reduce_partials<1>(r.part, r.nblocks, r.out, lds); break;
+    case 2: reduce_partials<2>(r.part, r.nblocks, r.out, lds); break;
+    case 3: reduce_partials<3>(r.part, r.nblocks, r.out, lds); break;
+    default: reduce_partials<4>(r.part, r.nblocks, r.out, lds);
   }
 }
 
@@ -116,17 +135,21 @@ __global__ __launch_bounds__(kBlock) void elementwise_kernel(int n, double* __re
 // Power iteration finalisers (one workgroup).
 __global__ __launch_bounds__(1024) void power_finalize_s2(const double* __restrict__ part, int nb, PowerState* st)
 {
-  __shared__ double lds[1024];
+  __shared__ double lds[1][1024];
   if (st->done != 0.0) return;
-  double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) s += part[b];
-  lds[threadIdx.x] = s;
-  __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) lds[threadIdx.x] += lds[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) st->s2 = lds[0];
+  reduce_partials<1>(part, nb, &st->s2, lds);
+}
+
+// Ends a power step: res and the next norm from the sums of squares (lane 0).
+__device__ inline void end_power_step(PowerState* st, double res2, double nrm2, double tol)
+{
+  const double res = sqrt(res2);
+  st->res          = res;
+  st->iters += 1.0;
+  if (res < tol)
+    st->done = 1.0;
+  else
+    st->nrm = sqrt(nrm2);
 }
 
 __global__ __launch_bounds__(1024) void power_finalize_res(const double* __restrict__ part,
@@ -135,31 +158,11 @@ __global__ __launch_bounds__(1024) void power_finalize_res(const double* __restr
                                                            double tol)
 {
   __shared__ double lds[2][1024];
+  __shared__ double sums[2];
   if (st->done != 0.0) return;
-  double s0 = 0.0, s1 = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    s0 += part[2 * (size_t)b];
-    s1 += part[2 * (size_t)b + 1];
-  }
-  lds[0][threadIdx.x] = s0;
-  lds[1][threadIdx.x] = s1;
+  reduce_partials<2>(part, nb, sums, lds);
   __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) {
-      lds[0][threadIdx.x] += lds[0][threadIdx.x + off];
-      lds[1][threadIdx.x] += lds[1][threadIdx.x + off];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    const double res = sqrt(lds[0][0]);
-    st->res          = res;
-    st->iters += 1.0;
-    if (res < tol)
-      st->done = 1.0;
-    else
-      st->nrm = sqrt(lds[1][0]);
-  }
+  if (threadIdx.x == 0) end_power_step(st, sums[0], sums[1], tol);
 }
 
 // Problems of at most kPowerSmallRows rows end a power step in one workgroup:
@@ -175,19 +178,14 @@ __global__ __launch_bounds__(1024) void power_step_small(const double* __restric
                                                          double tol)
 {
   __shared__ double lds[2][1024];
+  __shared__ double sums[2];
+  __shared__ double s2_lds;
   if (st->done != 0.0) return;
-  const int tid = threadIdx.x;
-  double s = 0.0;
-  for (int b = tid; b < nb; b += blockDim.x) s += part[b];
-  lds[0][tid] = s;
-  __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if (tid < off) lds[0][tid] += lds[0][tid + off];
-    __syncthreads();
-  }
-  const double s2  = lds[0][0];
+  const int tid    = threadIdx.x;
   const double nrm = st->nrm;
+  reduce_partials<1>(part, nb, &s2_lds, lds);
   __syncthreads();
+  const double s2 = s2_lds;
   double r2 = 0.0, z2 = 0.0;
   for (int i = tid; i < m; i += blockDim.x) {
     const double q = zold[i] / nrm;
@@ -198,22 +196,14 @@ __global__ __launch_bounds__(1024) void power_step_small(const double* __restric
   lds[0][tid] = r2;
   lds[1][tid] = z2;
   __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
-    if (tid < off) {
-      lds[0][tid] += lds[0][tid + off];
-      lds[1][tid] += lds[1][tid + off];
-    }
-    __syncthreads();
+  if (tid < 2 * kWave) {
+    const double v = tree_1024(lds[tid / kWave]);
+    if (tid % kWave == 0) sums[tid / kWave] = v;
   }
+  __syncthreads();
   if (tid == 0) {
-    st->s2           = s2;
-    const double res = sqrt(lds[0][0]);
-    st->res          = res;
-    st->iters += 1.0;
-    if (res < tol)
-      st->done = 1.0;
-    else
-      st->nrm = sqrt(lds[1][0]);
+    st->s2 = s2;
+    end_power_step(st, sums[0], sums[1], tol);
   }
 }
 
@@ -928,10 +918,17 @@ void launch_tiled(const MatStruct& M, const typename Epi::Mat* vals, double* red
                    epi, s, M.plan.fused ? M.plan.long_cnt.get() : nullptr);
 }
 
-void launch_reduce(const double* part, int nblocks, int nred, double* out, hipStream_t s,
-                   const double* skip = nullptr)
+void launch_reduce(const double* part, int nblocks, int nred, double* out, hipStream_t s)
 {
-  hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(1024), 0, s, part, nblocks, nred, out, skip);
+  const Reduction r{part, nblocks, nred, out};
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(1024), 0, s, r, r);
+  CUOPT_HIP_CHECK(hipGetLastError());
+}
+
+// Two reductions, of different partials, in one launch.
+void launch_reduce(const Reduction& a, const Reduction& b, hipStream_t s)
+{
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3(2), dim3(1024), 0, s, a, b);
   CUOPT_HIP_CHECK(hipGetLastError());
 }
 
@@ -1271,7 +1268,7 @@ class PdlpSolver {
 
   DevBuf<V> x_[2], y_[2], x0_, y0_, xbar_, ybar_, xhat_, yhat_, slack_, aty_;
   DevBuf<double> xu_, yu_, su_;
-  DevBuf<double> red_, scal_;
+  DevBuf<double> red_, red2_, scal_;  // red2_: partials of a pass over A^T that is reduced together with one over A
   DevBuf<double> rp_res_, rd_res_;          // per_constraint_residual: per-row / per-column residuals
   double linf_p_ = 0.0, linf_d_ = 0.0;
   DevBuf<double> best_x_, best_y_, best_s_;  // save_best_primal_so_far
@@ -1442,6 +1439,7 @@ void PdlpSolver<V>::setup_scaling()
   const int red_blocks = std::max({A_.plan.red_blocks(), AT_.plan.red_blocks(), ew_grid(std::max(m_, n_)),
                                    ew_grid(std::max(nnz, 1))});
   red_.resize((size_t)red_blocks * kMaxRed);
+  red2_.resize((size_t)AT_.plan.red_blocks() * kMaxRed);
   scal_.resize(S_COUNT);
   scal_.zero(stream_);
   Dr_.resize(m_);
@@ -1835,9 +1833,9 @@ void PdlpSolver<V>::evaluate_kkt(const Tolerances& tol)
   if (per && rp_res_.size() < (size_t)std::max(m_, 1)) rp_res_.resize(std::max(m_, 1));
   if (per && rd_res_.size() < (size_t)std::max(n_, 1)) rd_res_.resize(std::max(n_, 1));
   launch_tiled(A_, a_orig_.get(), red_.get(), kkt_rows(), stream_);
-  launch_reduce(red_.get(), A_.plan.red_blocks(), 3, scal_.get() + S_KKT_RP2, stream_);
-  launch_tiled(AT_, at_orig_.get(), red_.get(), kkt_cols(), stream_);
-  launch_reduce(red_.get(), AT_.plan.red_blocks(), 4, scal_.get() + S_KKT_RD2, stream_);
+  launch_tiled(AT_, at_orig_.get(), red2_.get(), kkt_cols(), stream_);
+  launch_reduce(Reduction{red_.get(), A_.plan.red_blocks(), 3, scal_.get() + S_KKT_RP2},
+                Reduction{red2_.get(), AT_.plan.red_blocks(), 4, scal_.get() + S_KKT_RD2}, stream_);
   if (per) {
     const int ab = st_.per_constraint_absolute;
     hipLaunchKernelGGL(linf_rel_kernel, dim3(1), dim3(1024), 0, stream_, rp_res_.get(), cb_orig_.get(), nullptr, m_,
@@ -1957,10 +1955,10 @@ void PdlpSolver<V>::launch_step(int j, bool major, bool fpe, double* ny_slot, do
 #undef CUOPT_DUAL
   if (ev_[2]) CUOPT_HIP_CHECK(hipEventRecord(ev_[2], stream_));
   if (fpe) {
-    launch_reduce(red_.get(), A_.plan.red_blocks(), 1, ny_slot, stream_);
-    launch_tiled(AT_, at_w_.get(), red_.get(), FpeEpi<V>{ybar_.get(), aty_.get(), xbar_.get(), x_[c].get()},
+    launch_tiled(AT_, at_w_.get(), red2_.get(), FpeEpi<V>{ybar_.get(), aty_.get(), xbar_.get(), x_[c].get()},
                  stream_);
-    launch_reduce(red_.get(), AT_.plan.red_blocks(), 2, fpe_slot, stream_);
+    launch_reduce(Reduction{red_.get(), A_.plan.red_blocks(), 1, ny_slot},
+                  Reduction{red2_.get(), AT_.plan.red_blocks(), 2, fpe_slot}, stream_);
   }
   cur_ = nx;
 }
@@ -2038,6 +2036,8 @@ SolveResult PdlpSolver<V>::run()
     const bool timed   = autotune_spmv<V>(A_, a_w_.get(), a_src_, stream_, st_.long_row_merge, false, ca);
     const bool timed_t = autotune_spmv<V>(AT_, at_w_.get(), ColSource{}, stream_, st_.long_row_merge, true, cat);
     CUOPT_HIP_CHECK(hipStreamSynchronize(stream_));
+    if (red_.size() < (size_t)A_.plan.red_blocks() * kMaxRed) red_.resize((size_t)A_.plan.red_blocks() * kMaxRed);
+    if (red2_.size() < (size_t)AT_.plan.red_blocks() * kMaxRed) red2_.resize((size_t)AT_.plan.red_blocks() * kMaxRed);
     if (timed || timed_t) R.info[CUOPT_AMD_INFO_TUNE_TIME] = elapsed() - t;
     R.info[CUOPT_AMD_INFO_LANES_BIAS_A]  = ca.bias;
     R.info[CUOPT_AMD_INFO_LANES_BIAS_AT] = cat.bias;

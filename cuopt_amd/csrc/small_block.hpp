@@ -421,23 +421,6 @@ inline size_t small_power_lds_bytes(int m, int n)
          64;
 }
 
-// Sum of a[0..1023] by lane 0 of one wavefront, in the order of power_step_small's tree.
-__device__ inline double small_tree_1024(const double* a)
-{
-  const int lane = threadIdx.x & (kWave - 1);
-  double s[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) s[i] = a[lane + kWave * i];
-#pragma unroll
-  for (int off = 8; off > 0; off >>= 1)
-#pragma unroll
-    for (int i = 0; i < off; ++i) s[i] += s[i + off];
-  double v = s[0];
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_down(v, off, kWave);
-  return v;
-}
-
 template <int R>
 __global__ __launch_bounds__(kSmallThreads) void small_power_kernel(SmallPowerArgs A)
 {
@@ -489,7 +472,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_power_kernel(SmallPowerAr
     all[kSmallThreads + tid] = z2;
     __syncthreads();
     if (tid < 2 * kWave) {
-      const double v = small_tree_1024(all + (tid / kWave) * kSmallThreads);
+      const double v = tree_1024(all + (tid / kWave) * kSmallThreads);
       if (tid % kWave == 0) sums[tid / kWave] = v;
     }
     __syncthreads();
