@@ -1125,17 +1125,15 @@ __global__ __launch_bounds__(BT, wg_per_cu(BT)) void batch_pdlp_kernel(BatchArgs
         zero_red(red);
 #define CUOPT_BPRIMAL(MAJ, FP)                                                                              \
   do {                                                                                                        \
-    PrimalStepEpi<V, MAJ, FP, true> e{ys[ci], xs[ci], c_w, bnd_w, xanc, xbar, xs[nx], xhat, slack, aty, &sc, jj,         \
-                                refine_active};                                                               \
-    e.begin();                                                                                               \
+    const OncePerPass<PrimalStepEpi<V, MAJ, FP>> e(PrimalStepEpi<V, MAJ, FP>{                                     \
+      ys[ci], xs[ci], c_w, bnd_w, xanc, xbar, xs[nx], xhat, slack, aty, &sc, jj, refine_active});                 \
     if (vec_in_lds) rows_pass<BT, 0>(tptr, tidx, tw, d.lgt, tblk, st, LdsGather<decltype(e)>{e, as_lds(ys[ci])}, red);  \
     else rows_pass<BT, 0>(tptr, tidx, tw, d.lgt, tblk, st, GlobalGather<decltype(e)>{e, as_global(ys[ci])}, red);        \
   } while (0)
 #define CUOPT_BDUAL(MAJ, FP)                                                                                 \
   do {                                                                                                        \
-    DualStepEpi<V, MAJ, FP, true> e{xbar, ys[ci], cb_w, yanc, ys[nx], yhat, ybar, &sc, jj,                               \
-                              refine_active ? (const V*)kink : nullptr};                                        \
-    e.begin();                                                                                               \
+    const OncePerPass<DualStepEpi<V, MAJ, FP>> e(DualStepEpi<V, MAJ, FP>{                                         \
+      xbar, ys[ci], cb_w, yanc, ys[nx], yhat, ybar, &sc, jj, refine_active ? (const V*)kink : nullptr});           \
     if (vec_in_lds) rows_pass<BT, (FP) ? 1 : 0>(aptr, aidx, aw, d.lga, ablk, st, LdsGather<decltype(e)>{e, as_lds((const V*)xbar)}, red); \
     else rows_pass<BT, (FP) ? 1 : 0>(aptr, aidx, aw, d.lga, ablk, st, GlobalGather<decltype(e)>{e, as_global((const V*)xbar)}, red); \
   } while (0)

@@ -108,11 +108,7 @@ __device__ inline double uniform_value(double v)
 }
 
 // ---- primal step over rows of A~^T (columns j): AtY, projection, reflection, Halpern.
-// HOIST (the batch kernel, many rows per lane): begin() sets the step's scalars once
-// per pass; without it each row evaluates them, which the tiled kernels overlap with
-// their memory accesses (evaluated before their first loads, they took the steps of
-// the 500 k x 1 M LP about 1 % longer).
-template <typename V, bool MAJOR, bool FPE, bool HOIST = false>
+template <typename V, bool MAJOR, bool FPE>
 struct PrimalStepEpi {
   using Mat = V;
   using Acc = typename AccFor<V>::type;
@@ -133,12 +129,6 @@ struct PrimalStepEpi {
   // Recentred (refined) solves: store only the part (x-hat - x) / tau of the slack; the
   // termination check adds the FP64 reduced cost of the corrected point.
   bool small_slack;
-  V htau = V(0), hw = V(0);
-  __device__ void begin()
-  {
-    htau = uniform_value((V)sc->tau);
-    hw   = uniform_value(halpern_weight<V>(sc, j));
-  }
   __device__ bool skip() const { return false; }
   struct Pre {
     V x, c, x0;
@@ -146,10 +136,13 @@ struct PrimalStepEpi {
   };
   __device__ typename Acc::Elem product(V v, int col, int) const { return Acc::prod(v, y[col]); }
   __device__ Pre load(int r) const { return Pre{x[r], c[r], x0[r], bnd[r]}; }
-  __device__ void row(int r, const Acc& aty, const Pre& p, double (&)[kMaxRed]) const
+  __device__ void row(int r, const Acc& aty, const Pre& p, double (&red)[kMaxRed]) const
   {
-    const V tau     = HOIST ? htau : (V)sc->tau;
-    const V w       = HOIST ? hw : halpern_weight<V>(sc, j);
+    row(r, aty, p, red, (V)sc->tau, halpern_weight<V>(sc, j));
+  }
+  __device__ V step_size() const { return (V)sc->tau; }
+  __device__ void row(int r, const Acc& aty, const Pre& p, double (&)[kMaxRed], V tau, V w) const
+  {
     const V next    = p.x - tau * aty.rsub(p.c);
     const V clamped = mx(mn(next, p.b.y), p.b.x);
     const V xb      = V(2) * clamped - p.x;
@@ -201,7 +194,7 @@ struct TilePipelining<PrimalStepEpi<double, MAJOR, FPE>, TILE> {
 };
 
 // ---- dual step over rows of A~ (rows i): A x-bar, projection, reflection, Halpern.
-template <typename V, bool MAJOR, bool FPE, bool HOIST = false>
+template <typename V, bool MAJOR, bool FPE>
 struct DualStepEpi {
   using Mat = V;
   using Acc = typename AccFor<V>::type;
@@ -220,12 +213,6 @@ struct DualStepEpi {
   // dual objective term, which sits at y = 0 in the original problem and at
   // -Dd * y* / Dr in the coordinates of a correction problem.
   const V* kink;
-  V hsigma = V(0), hw = V(0);  // HOIST: set by begin(), as in the primal step
-  __device__ void begin()
-  {
-    hsigma = uniform_value((V)sc->sigma);
-    hw     = uniform_value(halpern_weight<V>(sc, j));
-  }
   __device__ bool skip() const { return false; }
   struct Pre {
     V y, y0, k;
@@ -235,8 +222,11 @@ struct DualStepEpi {
   __device__ Pre load(int r) const { return Pre{y[r], y0[r], kink ? kink[r] : V(0), cb[r]}; }
   __device__ void row(int r, const Acc& ax, const Pre& p, double (&red)[kMaxRed]) const
   {
-    const V sigma = HOIST ? hsigma : (V)sc->sigma;
-    const V w     = HOIST ? hw : halpern_weight<V>(sc, j);
+    row(r, ax, p, red, (V)sc->sigma, halpern_weight<V>(sc, j));
+  }
+  __device__ V step_size() const { return (V)sc->sigma; }
+  __device__ void row(int r, const Acc& ax, const Pre& p, double (&red)[kMaxRed], V sigma, V w) const
+  {
     V nd;
     if (kink) {
       // The projection of the original problem moved to the kink k, written as
@@ -258,6 +248,25 @@ struct DualStepEpi {
       red[0] += d * d;
     }
     ynext[r] = w * yb + (V(1) - w) * p.y0;
+  }
+};
+
+// A step epilogue whose scalars are evaluated once per pass instead of once per row (the
+// FP64 division of the Halpern weight was most of a row's epilogue): for kernels
+// whose lanes take many rows.  The tiled kernels overlap it with their memory accesses;
+// evaluated before their first loads, it took the steps of the 500 k x 1 M LP about
+// 1 % longer.
+template <class Base, typename V = typename Base::Mat>
+struct OncePerPass : Base {
+  V step, weight;
+  __device__ explicit OncePerPass(const Base& b)
+    : Base(b), step(uniform_value(b.step_size())), weight(uniform_value(halpern_weight<V>(b.sc, b.j)))
+  {
+  }
+  __device__ OncePerPass(const Base& b, V s, V w) : Base(b), step(s), weight(w) {}
+  __device__ void row(int r, const typename Base::Acc& sum, const typename Base::Pre& p, double (&red)[kMaxRed]) const
+  {
+    Base::row(r, sum, p, red, step, weight);
   }
 };
 

@@ -331,14 +331,15 @@ __global__ __launch_bounds__(kSmallThreads) void small_block_kernel(SmallArgs<V>
       __syncthreads();
     }
     auto primal = [&](auto MAJ, auto FP) {
-      PrimalStepEpi<V, decltype(MAJ)::value, decltype(FP)::value, true> e{
-        y, x, c, bnd, x0, xbar, x, A.xhat, A.slack, A.aty, &A.sc, s, A.refine, (V)A.sc.tau, weight[s]};
-      small_pass<decltype(e), R, true>(MT, A.tidx, A.tw, st, prod, e, part, red_lds);
+      using E = PrimalStepEpi<V, decltype(MAJ)::value, decltype(FP)::value>;
+      const OncePerPass<E> e(E{y, x, c, bnd, x0, xbar, x, A.xhat, A.slack, A.aty, nullptr, s, A.refine}, (V)A.sc.tau,
+                             weight[s]);
+      small_pass<OncePerPass<E>, R, true>(MT, A.tidx, A.tw, st, prod, e, part, red_lds);
     };
     auto dual = [&](auto MAJ, auto FP) {
-      DualStepEpi<V, decltype(MAJ)::value, decltype(FP)::value, true> e{
-        xbar, y, cb, y0, y, A.yhat, A.ybar, &A.sc, s, A.kink, (V)A.sc.sigma, weight[s]};
-      small_pass<decltype(e), R, true>(MA, A.aidx, A.aw, sa, prod, e, part, red_lds);
+      using E = DualStepEpi<V, decltype(MAJ)::value, decltype(FP)::value>;
+      const OncePerPass<E> e(E{xbar, y, cb, y0, y, A.yhat, A.ybar, nullptr, s, A.kink}, (V)A.sc.sigma, weight[s]);
+      small_pass<OncePerPass<E>, R, true>(MA, A.aidx, A.aw, sa, prod, e, part, red_lds);
     };
     using std::false_type;
     using std::true_type;
