@@ -919,3 +919,21 @@ def test_small_lp_in_one_workgroup_is_the_tiled_solve(monkeypatch, lp, prec):
             assert np.array_equal(getattr(a, f), getattr(b, f), equal_nan=True), (kw, f)
         for k in ("eta0", "power_iterations", "omega", "restarts", "checks", "refine_rounds", "gap"):
             assert a.info[k] == b.info[k], (kw, k)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+@pytest.mark.parametrize("limit", [10, 20, 195, 200, 210, 990, 1100])
+def test_steps_launched_before_their_check_leave_its_point(monkeypatch, limit, prec):
+    # The steps after a check between restarts are launched before its result is known
+    # (only where they are replayed as a graph); a solve that the check ends, at the
+    # limit or at the tolerance, returns the check's own point, bit for bit.
+    lp = G.random_lp(m=900, n=2300, seed=6)
+    for kw in (dict(tol=0.0), dict(tol=3e-2), dict(tol=0.0, params={"save_best_primal_so_far": 1})):
+        got = []
+        for graphs in ("0", "1"):
+            monkeypatch.setenv("CUOPT_AMD_GRAPHS", graphs)
+            got.append(c_api.solve(lp, precision=prec, iteration_limit=limit, time_limit=60.0, **kw))
+        a, b = got
+        assert (a.status, a.iterations) == (b.status, b.iterations), kw
+        for f in ("x", "y", "reduced_cost", "trace"):
+            assert np.array_equal(getattr(a, f), getattr(b, f), equal_nan=True), (kw, f)
