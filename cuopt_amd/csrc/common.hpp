@@ -8,7 +8,10 @@
 #include <cstdio>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
+
+#include "dev_pool.hpp"
 
 namespace cuopt_amd {
 
@@ -26,7 +29,7 @@ struct hip_error : std::runtime_error {
     }                                                                                       \
   } while (0)
 
-// Owning device allocation (hipMalloc / hipFree), move-only.
+// Owning device allocation (hipMalloc / hipFree, or a solve's lease: dev_pool.hpp), move-only.
 template <typename T>
 class DevBuf {
  public:
@@ -35,29 +38,42 @@ class DevBuf {
   ~DevBuf() { release(); }
   DevBuf(const DevBuf&)            = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr; o.n_ = 0; }
+  DevBuf(DevBuf&& o) noexcept
+    : p_(std::exchange(o.p_, nullptr)), n_(std::exchange(o.n_, 0)), lease_(std::exchange(o.lease_, nullptr)),
+      block_(o.block_)
+  {
+  }
   DevBuf& operator=(DevBuf&& o) noexcept
   {
     if (this != &o) {
       release();
-      p_ = o.p_;
-      n_ = o.n_;
-      o.p_ = nullptr;
-      o.n_ = 0;
+      p_     = std::exchange(o.p_, nullptr);
+      n_     = std::exchange(o.n_, 0);
+      lease_ = std::exchange(o.lease_, nullptr);
+      block_ = o.block_;
     }
     return *this;
   }
   void resize(size_t n)
   {
     release();
-    if (n) CUOPT_HIP_CHECK(hipMalloc(&p_, n * sizeof(T)));
+    const PoolLease::Current& c = PoolLease::current();
+    if (c.lease && n * sizeof(T) >= kPoolMin) {
+      CUOPT_HIP_CHECK(c.lease->alloc(n * sizeof(T), c.stream, block_));
+      p_     = static_cast<T*>(block_.p);
+      lease_ = c.lease;
+    } else if (n) {
+      CUOPT_HIP_CHECK(hipMalloc(&p_, n * sizeof(T)));
+    }
     n_ = n;
   }
   void release()
   {
-    if (p_) (void)hipFree(p_);
-    p_ = nullptr;
-    n_ = 0;
+    if (lease_) lease_->release(block_);
+    else if (p_) (void)hipFree(p_);
+    p_     = nullptr;
+    n_     = 0;
+    lease_ = nullptr;
   }
   T* get() const { return p_; }
   size_t size() const { return n_; }
@@ -80,6 +96,8 @@ class DevBuf {
  private:
   T* p_     = nullptr;
   size_t n_ = 0;
+  PoolLease* lease_ = nullptr;  // where block_ goes back to
+  PoolBlock block_;
 };
 
 // Device arrays carved from one allocation: one hipMalloc and one hipFree for a

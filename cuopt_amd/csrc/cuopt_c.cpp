@@ -37,6 +37,7 @@ namespace {
 
 struct ProblemHandle {
   LpHost lp;
+  PoolUser keeps_pool;
 };
 
 struct SettingsHandle {
@@ -47,6 +48,7 @@ struct SettingsHandle {
   cuOptMIPSetSolutionCallback mip_set_cb = nullptr;
   void* mip_get_data = nullptr;
   void* mip_set_data = nullptr;
+  PoolUser keeps_pool;
 };
 
 struct SolutionHandle {

@@ -1149,7 +1149,8 @@ class PdlpSolver {
 
   ~PdlpSolver()
   {
-    if (stream_) (void)hipStreamSynchronize(stream_);  // steps launched ahead may still run
+    // steps launched ahead may still run
+    if (stream_ && hipStreamSynchronize(stream_) != hipSuccess) lease_.drop();
     for (auto& g : graphs_) (void)hipGraphExecDestroy(g.second);
     if (checked_) (void)hipEventDestroy(checked_);
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -1221,6 +1222,7 @@ class PdlpSolver {
   const int m_, n_;
   clock::time_point t0_;
   hipStream_t stream_ = nullptr;
+  PoolLease lease_;  // ends after the arrays below
   double* h_scal_     = nullptr;
   PowerState* h_power_ = nullptr;
 
@@ -2021,6 +2023,7 @@ SolveResult PdlpSolver<V>::run()
   SolveResult R;
   t0_ = clock::now();
   CUOPT_HIP_CHECK(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+  const PoolLease::Scope from_lease(lease_, stream_);
   CUOPT_HIP_CHECK(hipHostMalloc((void**)&h_scal_, S_COUNT * sizeof(double), hipHostMallocDefault));
   if (const char* g = std::getenv("CUOPT_AMD_GRAPHS")) use_graphs_ = std::atoi(g) != 0;
   obj_sf_  = lp_.maximize ? -1.0 : 1.0;

@@ -937,3 +937,41 @@ def test_steps_launched_before_their_check_leave_its_point(monkeypatch, limit, p
         assert (a.status, a.iterations) == (b.status, b.iterations), kw
         for f in ("x", "y", "reduced_cost", "trace"):
             assert np.array_equal(getattr(a, f), getattr(b, f), equal_nan=True), (kw, f)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_memory_kept_between_solves(prec):
+    # Solves that take memory earlier solves left, of other sizes and precisions and on
+    # other threads, give the results of a solve in new memory; with the last handle the
+    # memory is given back.
+    import concurrent.futures
+    import gc
+
+    import torch
+
+    def solve(lp, p):
+        prob, conf = c_api.Problem(lp), c_api.make_settings(1e-3, p, 300, 60.0)
+        return c_api.solve_problem(prob, conf)
+
+    def alive():
+        gc.collect()
+        return any(isinstance(o, (c_api.Problem, c_api.SolverSettings)) for o in gc.get_objects())
+
+    lps = [G.skewed_lp(m=30000, n=70000, seed=1), G.skewed_lp(m=40000, n=80000, seed=2),
+           G.random_lp(m=35000, n=33000, seed=3)]
+    first = [solve(lp, prec) for lp in lps]
+    keeps_alive = alive()
+    free = torch.cuda.mem_get_info()[0]
+    kept = c_api.SolverSettings()
+    other = "fp64" if prec == "fp32_mixed" else "fp32_mixed"
+    solve(lps[1], other)
+    again = [solve(lp, prec) for lp in lps]
+    with concurrent.futures.ThreadPoolExecutor(3) as pool:
+        again += list(pool.map(lambda lp: solve(lp, prec), lps + lps[::-1]))
+    for a, b in zip(first + first + first[::-1], again):
+        assert a.iterations == b.iterations
+        for f in ("x", "y", "reduced_cost"):
+            assert np.array_equal(getattr(a, f), getattr(b, f)), f
+    del kept
+    if not keeps_alive and not alive():
+        assert torch.cuda.mem_get_info()[0] >= free - (16 << 20)
