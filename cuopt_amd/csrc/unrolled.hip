@@ -69,7 +69,13 @@ inline int slab_width(Shape s)
   return s == Shape::k4x1 ? 4 : s == Shape::k8x1 ? 8 : s == Shape::k8x4 ? 32 : 16;
 }
 
-// The shape of a call.  Up to 4 members: 4 lanes to a row.  Otherwise the least
+// The shape of a call.  Up to 4 members: 8 lanes to a row up to kFewRows rows and columns,
+// where a row's chain of loads sets the time and eight lanes read it in fewer rounds, and 4
+// lanes above.  207 steps with gradients in FP64, ms, by shape 4x1 / 8x1 (and the kernel
+// of one row per wavefront): 1 104 x 2 760, B 1 5.04 / 4.87 (4.96); 2 000 x 5 000, B 2 5.53 / 5.07
+// (5.55); 5 500 x 13 750, B 4 6.13 / 5.95 (9.86); 8 000 x 20 000, B 1 6.46 / 6.64 (12.3).  Only the
+// smallest lost to one row per wavefront (200 x 500, B 1 4.62 in either against 4.43).
+// More members: the least
 // (members computed, those past B included) x (cost per member) among the shapes that
 // leave at least kMinWaves wavefronts (one member per lane always may).  Measured, ms,
 // by shape 8x1 / 16x1 / 8x2 / 8x4 (the kernel of one row per wavefront in brackets):
@@ -81,6 +87,7 @@ inline int slab_width(Shape s)
 //   FP64 16 000 x 40 000, B 12, 200 steps with gradients    12.9 / 12.5 / 11.2        (21.3)
 //   FP64  5 000 x 12 500, B 24, 200 steps with gradients    7.61 / 9.69 / 8.59        (10.6)
 constexpr long long kMinWaves = 1200;
+constexpr int kFewRows        = 16384;
 
 template <typename V>
 Shape pick_shape(int m, int n, int B)
@@ -91,6 +98,7 @@ Shape pick_shape(int m, int n, int B)
       if (v == (s == Shape::k4x1 ? 41 : s == Shape::k8x1 ? 81 : s == Shape::k16x1 ? 161 : s == Shape::k8x2 ? 82 : 84))
         return s == Shape::k8x4 && sizeof(V) == 8 ? Shape::k8x2 : s;
   }
+  if (B <= 4) return std::max(m, n) <= kFewRows ? Shape::k8x1 : Shape::k4x1;
   Shape best  = Shape::k4x1;
   double cost = 1e300;
   struct Option {
@@ -101,7 +109,7 @@ Shape pick_shape(int m, int n, int B)
   for (const Option& o : {Option{Shape::k8x1, 1, 1.15}, Option{Shape::k16x1, 1, 1.0}, Option{Shape::k8x2, 2, 0.95},
                           Option{Shape::k8x4, 4, 0.9}}) {
     const long long W = slab_width(o.s), members = (B + W - 1) / W * W;
-    if (B <= 4 || o.vw * sizeof(V) > 16) continue;
+    if (o.vw * sizeof(V) > 16) continue;
     if (o.vw > 1 && (long long)std::min(m, n) * members / (kWave * o.vw) < kMinWaves) continue;
     if ((unsigned long long)std::max(m, n) * W * sizeof(V) >= (1ULL << 32)) continue;  // 32-bit gather offsets
     if (members * o.per_member < cost) {
