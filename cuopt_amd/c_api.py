@@ -372,6 +372,11 @@ def solve(lp, tol: float = 1e-4, precision: str = "fp64", iteration_limit: int |
     return solve_problem(prob, s)
 
 
+def release_memory() -> None:
+    """Frees the device memory that finished solves left for the next ones."""
+    lib().cuOptAmdReleaseMemory()
+
+
 def batch_solve(lps, tol: float = 1e-4, precision: str = "fp64", iteration_limit: int | None = None,
                 time_limit: float | None = None, **params) -> list[Result]:
     """cuOptAmdBatchSolve over ``lps`` (LP objects or already built ``Problem`` handles): one

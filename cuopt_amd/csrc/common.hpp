@@ -63,7 +63,7 @@ class DevBuf {
       p_     = static_cast<T*>(block_.p);
       lease_ = c.lease;
     } else if (n) {
-      CUOPT_HIP_CHECK(hipMalloc(&p_, n * sizeof(T)));
+      CUOPT_HIP_CHECK(pool_malloc(reinterpret_cast<void**>(&p_), n * sizeof(T)));
     }
     n_ = n;
   }

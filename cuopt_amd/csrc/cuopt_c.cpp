@@ -37,7 +37,6 @@ namespace {
 
 struct ProblemHandle {
   LpHost lp;
-  PoolUser keeps_pool;
 };
 
 struct SettingsHandle {
@@ -48,7 +47,6 @@ struct SettingsHandle {
   cuOptMIPSetSolutionCallback mip_set_cb = nullptr;
   void* mip_get_data = nullptr;
   void* mip_set_data = nullptr;
-  PoolUser keeps_pool;
 };
 
 struct SolutionHandle {
@@ -644,6 +642,8 @@ cuopt_int_t cuOptSolve(cuOptOptimizationProblem problem, cuOptSolverSettings set
   *solution_ptr = sol;
   return R.error;
 }
+
+void cuOptAmdReleaseMemory(void) { PoolStore::get().trim(); }
 
 cuopt_int_t cuOptAmdBatchSolve(cuopt_int_t num_problems,
                                const cuOptOptimizationProblem* problems,

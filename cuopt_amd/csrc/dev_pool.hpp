@@ -9,9 +9,11 @@
 // released array goes back to the lease and may serve a later one: all of a solve's work
 // is on one stream, so the order of the launches orders the uses too.  When the solve
 // ends (its stream is idle) the lease hands its blocks to a process-wide store, which
-// keeps at most kPoolCap bytes, the oldest freed first; the store is emptied when no
-// problem or settings handle is left, and when an allocation fails.  Contents are never
-// reused: an array from the store is as undefined as one from hipMalloc.
+// keeps at most kPoolCap bytes, the oldest freed first, and none that the last kPoolAge
+// solves left unused; it is emptied by cuOptAmdReleaseMemory and when an allocation
+// fails.  It outlives the handles: freeing with the last of them would only move the cost
+// to a caller that makes its handles anew for each solve.  Contents are never reused:
+// an array from the store is as undefined as one from hipMalloc.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -24,11 +26,13 @@ namespace cuopt_amd {
 
 constexpr size_t kPoolMin = 256 << 10;    // below it hipFree takes a few microseconds
 constexpr size_t kPoolCap = 2ull << 30;   // under 1 % of the card's memory; 4 GiB was no faster at 1 M x 2 M
+constexpr long kPoolAge   = 8;           // solves that an unused block is kept for
 
 struct PoolBlock {
   void* p      = nullptr;
   size_t bytes = 0;
   int dev      = 0;
+  long solve   = 0;  // the solve that gave it to the store
 };
 
 // Whether a block of `have` bytes may serve a request of `want`: at most a quarter is unused.
@@ -73,9 +77,13 @@ class PoolStore {
     std::list<PoolBlock> out;
     {
       std::lock_guard<std::mutex> lock(mu_);
-      for (const PoolBlock& b : blocks) held_ += b.bytes;
+      ++solves_;
+      for (PoolBlock& b : blocks) {
+        held_ += b.bytes;
+        b.solve = solves_;
+      }
       blocks_.splice(blocks_.end(), blocks);
-      while (!blocks_.empty() && (held_ > kPoolCap || users_ == 0)) {
+      while (!blocks_.empty() && (held_ > kPoolCap || blocks_.front().solve + kPoolAge < solves_)) {
         held_ -= blocks_.front().bytes;
         out.splice(out.end(), blocks_, blocks_.begin());
       }
@@ -92,35 +100,25 @@ class PoolStore {
     }
     pool_free(out);
   }
-  void add_user()
-  {
-    std::lock_guard<std::mutex> lock(mu_);
-    ++users_;
-  }
-  void drop_user()
-  {
-    bool last = false;
-    {
-      std::lock_guard<std::mutex> lock(mu_);
-      last = --users_ == 0;
-    }
-    if (last) trim();
-  }
 
  private:
   std::mutex mu_;
   std::list<PoolBlock> blocks_;  // oldest first
   size_t held_ = 0;
-  long users_  = 0;
+  long solves_ = 0;
 };
 
-// A handle whose owner may solve (again): while there is one, the store keeps its blocks.
-struct PoolUser {
-  PoolUser() { PoolStore::get().add_user(); }
-  ~PoolUser() { PoolStore::get().drop_user(); }
-  PoolUser(const PoolUser&)            = delete;
-  PoolUser& operator=(const PoolUser&) = delete;
-};
+// hipMalloc, tried again with an emptied store if it fails.
+inline hipError_t pool_malloc(void** p, size_t bytes)
+{
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    PoolStore::get().trim();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
 
 // The blocks of one solve.  It outlives every array that took from it, and its stream is
 // idle when it ends.
@@ -146,12 +144,11 @@ class PoolLease {
     if (b.p) return hipSuccess;
     b.bytes      = bytes;
     b.dev        = dev;
-    hipError_t e = hipMalloc(&b.p, bytes);
-    if (e == hipErrorOutOfMemory) {
+    hipError_t e = pool_malloc(&b.p, bytes);
+    if (e == hipErrorOutOfMemory && !free_.empty()) {
       (void)hipGetLastError();
       (void)hipStreamSynchronize(s);
       pool_free(free_);
-      PoolStore::get().trim();
       e = hipMalloc(&b.p, bytes);
     }
     if (e != hipSuccess) b = PoolBlock{};

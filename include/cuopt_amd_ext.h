@@ -323,6 +323,10 @@ cuopt_int_t cuOptAmdBatchSolve(cuopt_int_t num_problems,
                                cuOptSolverSettings settings,
                                cuOptSolution* solutions);
 
+/* Frees the device memory kept from finished solves for the next ones (at most 2 GiB
+ * a process).  It is safe at any time, solves on other threads included. */
+void cuOptAmdReleaseMemory(void);
+
 #ifdef __cplusplus
 }
 #endif

@@ -942,10 +942,8 @@ def test_steps_launched_before_their_check_leave_its_point(monkeypatch, limit, p
 @pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
 def test_memory_kept_between_solves(prec):
     # Solves that take memory earlier solves left, of other sizes and precisions and on
-    # other threads, give the results of a solve in new memory; with the last handle the
-    # memory is given back.
+    # other threads, give the results of a solve in new memory; it is given back on request.
     import concurrent.futures
-    import gc
 
     import torch
 
@@ -953,16 +951,14 @@ def test_memory_kept_between_solves(prec):
         prob, conf = c_api.Problem(lp), c_api.make_settings(1e-3, p, 300, 60.0)
         return c_api.solve_problem(prob, conf)
 
-    def alive():
-        gc.collect()
-        return any(isinstance(o, (c_api.Problem, c_api.SolverSettings)) for o in gc.get_objects())
-
     lps = [G.skewed_lp(m=30000, n=70000, seed=1), G.skewed_lp(m=40000, n=80000, seed=2),
            G.random_lp(m=35000, n=33000, seed=3)]
-    first = [solve(lp, prec) for lp in lps]
-    keeps_alive = alive()
+    first = []
+    for lp in lps:
+        c_api.release_memory()
+        first.append(solve(lp, prec))
+    c_api.release_memory()
     free = torch.cuda.mem_get_info()[0]
-    kept = c_api.SolverSettings()
     other = "fp64" if prec == "fp32_mixed" else "fp32_mixed"
     solve(lps[1], other)
     again = [solve(lp, prec) for lp in lps]
@@ -972,6 +968,5 @@ def test_memory_kept_between_solves(prec):
         assert a.iterations == b.iterations
         for f in ("x", "y", "reduced_cost"):
             assert np.array_equal(getattr(a, f), getattr(b, f)), f
-    del kept
-    if not keeps_alive and not alive():
-        assert torch.cuda.mem_get_info()[0] >= free - (16 << 20)
+    c_api.release_memory()
+    assert torch.cuda.mem_get_info()[0] >= free - (16 << 20)
