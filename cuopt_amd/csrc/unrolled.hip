@@ -768,9 +768,10 @@ void forward_impl(UnrolledImpl& U, const double* c, const double* lc, const doub
   Views<V> M     = views<V>(U);
   const size_t members = (size_t)U.W * U.slabs, nB = U.n * members, mB = U.m * members;
   if (!U.seg.get()) U.seg.resize(1);
-  // The captured graphs hold the work buffer's addresses and the shapes.
-  const std::vector<long long> key{(long long)(uintptr_t)U.work.get(), U.B, U.every, U.ldb, (long long)sizeof(V),
-                                   (long long)U.shape};
+  // The captured graphs hold the work buffer's addresses and the shapes.  Where carve()
+  // places the checkpoints and all that follows them goes by the number of segments.
+  const std::vector<long long> key{(long long)(uintptr_t)U.work.get(), U.B, nseg, U.every, U.ldb,
+                                   (long long)sizeof(V), (long long)U.shape};
   if (key != U.graph_key) {
     U.drop_graphs();
     U.graph_key = key;

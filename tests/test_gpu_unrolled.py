@@ -325,3 +325,28 @@ def test_member_result_does_not_depend_on_the_slab_shape(monkeypatch, prec, per_
             for k, v in enumerate(run(list(range(B)))):
                 for i in range(B):
                     assert np.array_equal(v[i], alone[i][k][0]), (shape, B, k, i)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_one_handle_runs_other_numbers_of_steps(prec):
+    # A handle whose calls take 100, 60, 100, 23 and 172 steps of the same batch and checkpoint
+    # interval: its segment graphs and its working storage follow the call, so every
+    # point and gradient is that of a handle made for the call, bit for bit.
+    lp, _ = problem(6, m=200, n=500)
+    B, every = 8, 9
+    rng = np.random.default_rng(6)
+    c0 = lp.c[None, :] + 0.1 * rng.normal(size=(B, lp.n))
+    gx, gy = (torch.tensor(rng.normal(size=(B, k)), device=DEV) for k in (lp.n, lp.m))
+
+    def run(op):
+        c, b = (torch.tensor(v, device=DEV, requires_grad=True) for v in (c0, lp.con_lb))
+        x, y = op(c, b)
+        torch.autograd.backward([x, y], [gx, gy])
+        return [v.detach().cpu().numpy() for v in (x, y, c.grad, b.grad)]
+
+    kept = UnrolledPDHG(lp, ridge=1e-3, steps=100, checkpoint_every=every, precision=prec)
+    for steps in (100, 60, 100, 23, 172, 60):
+        kept.steps = steps
+        fresh = UnrolledPDHG(lp, ridge=1e-3, steps=steps, checkpoint_every=every, precision=prec)
+        for name, u, v in zip(("x", "y", "gc", "gb"), run(kept), run(fresh)):
+            assert np.array_equal(u, v), (steps, name)
