@@ -111,10 +111,10 @@ class _UnrolledFn(torch.autograd.Function):
         x = torch.empty(op.n, B, dtype=torch.float64, device=dev)
         y = torch.empty(op.m, B, dtype=torch.float64, device=dev)
         stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        op._generation += 1  # from here on the earlier checkpoints are gone, also if the call fails
         rc = _lib().cuOptAmdUnrolledForward(op.handle, B, op.steps, op.every, _ptr(c_nb), _ptr(lc_d), _ptr(uc_d),
                                              int(per_batch), _ptr(x), _ptr(y), stream)
         c_api._check(rc, "cuOptAmdUnrolledForward")
-        op._generation += 1
         ctx.op, ctx.generation, ctx.per_batch, ctx.B = op, op._generation, per_batch, B
         return x.t(), y.t()
 

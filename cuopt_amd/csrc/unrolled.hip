@@ -617,7 +617,8 @@ struct UnrolledImpl {
   DevBuf<float> aval32, tval32;
   DevBuf<double> lb64, ub64;
   DevBuf<float> lb32, ub32;
-  // last forward
+  // last forward; ready: it was queued whole, and its checkpoints stand in `work`
+  bool ready = false;
   int B = 0, K = 0, every = 1, ldb = 0;
   Shape shape = Shape::k4x1;
   int W = 4, slabs = 0;  // members per slab, slabs
@@ -1021,6 +1022,7 @@ void unrolled_forward(UnrolledHandle* h, int B, int K, int every, const double* 
 {
   auto* U = reinterpret_cast<UnrolledImpl*>(h);
   if (B <= 0 || K < 0 || every <= 0) throw validation_error("batch and checkpoint interval must be positive");
+  U->ready = false;  // a call that fails (its working storage may not fit) leaves nothing to differentiate
   U->B     = B;
   U->K     = K;
   U->every = every;
@@ -1034,13 +1036,14 @@ void unrolled_forward(UnrolledHandle* h, int B, int K, int every, const double* 
     forward_impl<float>(*U, c, lc, uc, x, y, s);
   else
     forward_impl<double>(*U, c, lc, uc, x, y, s);
+  U->ready = true;
 }
 
 void unrolled_backward(UnrolledHandle* h, const double* gx, const double* gy, double* gc, double* glc, double* guc,
                        void* stream)
 {
   auto* U = reinterpret_cast<UnrolledImpl*>(h);
-  if (U->B <= 0) throw validation_error("backward called before forward");
+  if (!U->ready) throw validation_error("backward called without a completed forward");
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (U->K == 0) {
     const size_t nB = (size_t)U->n * U->B, mB = (size_t)U->m * U->B;

@@ -350,3 +350,46 @@ def test_one_handle_runs_other_numbers_of_steps(prec):
         fresh = UnrolledPDHG(lp, ridge=1e-3, steps=steps, checkpoint_every=every, precision=prec)
         for name, u, v in zip(("x", "y", "gc", "gb"), run(kept), run(fresh)):
             assert np.array_equal(u, v), (steps, name)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_backward_after_a_forward_that_did_not_fit(prec):
+    # A forward whose working storage cannot be allocated fails, and so does the backward
+    # of any forward before it, through autograd and through the C entry point: the
+    # checkpoints are gone.  The handle works on.
+    import ctypes
+
+    from cuopt_amd import autograd, c_api
+
+    lp, _ = problem(7, m=60, n=150)
+    B = 3
+    rng = np.random.default_rng(7)
+    c0 = lp.c[None, :] + 0.1 * rng.normal(size=(B, lp.n))
+    op = UnrolledPDHG(lp, ridge=1e-3, steps=20, checkpoint_every=6, precision=prec)
+
+    def forward():
+        c, b = (torch.tensor(v, device=DEV, requires_grad=True) for v in (c0, lp.con_lb))
+        return c, (op(c, b)[0] ** 2).sum()
+
+    def native_backward():
+        gx, gc = (torch.ones(lp.n, B, dtype=torch.float64, device=DEV) for _ in range(2))
+        glc, guc = (torch.ones(lp.m, B, dtype=torch.float64, device=DEV) for _ in range(2))
+        args = [ctypes.c_void_p(t.data_ptr() if t is not None else None) for t in (gx, None, gc, glc, guc)]
+        rc = autograd._lib().cuOptAmdUnrolledBackward(op.handle, *args, None)
+        torch.cuda.synchronize()
+        return rc
+
+    c, loss = forward()
+    loss.backward(retain_graph=True)
+    first = c.grad.clone()
+    assert native_backward() == c_api.CUOPT_SUCCESS
+    op.every = 10 ** 9  # segment states for so many steps: terabytes
+    with pytest.raises(c_api.CuOptError):
+        forward()
+    op.every = 6
+    with pytest.raises(RuntimeError):
+        loss.backward()
+    assert native_backward() != c_api.CUOPT_SUCCESS
+    c, loss = forward()
+    loss.backward()
+    assert torch.equal(c.grad, first)
