@@ -146,14 +146,17 @@ struct MatView {
   int rows;
 };
 
-// The kXcds XCDs take the workgroups of a launch in turn.
-constexpr int kXcds = 8;
+// The kXcds XCDs take the workgroups of a launch in turn.  They lie in rows of at most
+// 2^kGridShift: a row of 2^24 would have 2^32 lanes, more than a launch can count.
+constexpr int kXcds      = 8;
+constexpr int kGridShift = 20;
 
 template <class L>
 dim3 slab_grid(int rows, int slabs)
 {
   const long long items = (long long)((std::max(rows, 1) + L::rows_per_wg - 1) / L::rows_per_wg) * slabs;
-  return dim3((unsigned)((items + kXcds - 1) / kXcds * kXcds));
+  const long long all = (items + kXcds - 1) / kXcds * kXcds, row = 1LL << kGridShift;
+  return dim3((unsigned)std::min(all, row), (unsigned)((all + row - 1) / row));
 }
 
 // This lane's slab, row and first member within the slab; false past the end.
@@ -165,8 +168,9 @@ __device__ inline bool my_place(int rows, int slabs, const int4* __restrict__ ru
 {
   const int blocks = (rows + L::rows_per_wg - 1) / L::rows_per_wg;
   const int items = blocks * slabs, per = (items + kXcds - 1) / kXcds;
-  const int item = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
-  if ((int)(blockIdx.x / kXcds) >= per || item >= items) return false;
+  const int at   = (int)(blockIdx.y << kGridShift) + (int)blockIdx.x;
+  const int item = at % kXcds * per + at / kXcds;
+  if (at / kXcds >= per || item >= items) return false;
   p.slab        = item / blocks;
   const int pos = (item - p.slab * blocks) * L::rows_per_wg + (int)threadIdx.x / L::LW;
   if (pos >= rows) return false;

@@ -393,3 +393,28 @@ def test_backward_after_a_forward_that_did_not_fit(prec):
     c, loss = forward()
     loss.backward()
     assert torch.equal(c.grad, first)
+
+
+def test_more_workgroups_than_one_grid_dimension_counts():
+    # One row, one column and 2^28 + 64 members: more than 2^24 workgroups of 256 lanes.  One
+    # step from x = 0, y = 0 has a closed form.
+    B, lam = (1 << 28) + 64, 1e-3
+    if torch.cuda.mem_get_info()[0] < (150 << 30):
+        pytest.skip("needs 150 GB of device memory")
+    lp = G.LP(m=1, n=1, row_offsets=np.array([0, 1], np.int32), col_indices=np.zeros(1, np.int32), values=np.ones(1),
+              c=np.ones(1), con_lb=np.ones(1), con_ub=np.ones(1), var_lb=np.zeros(1), var_ub=np.full(1, 5.0))
+    op = UnrolledPDHG(lp, ridge=lam, steps=1, checkpoint_every=1, precision="fp64")
+    eta = op.step_size
+    c = torch.linspace(-6.0, 1.0, B, dtype=torch.float64, device=DEV)[:, None].requires_grad_(True)
+    b = torch.ones(1, dtype=torch.float64, device=DEV)
+    x, y = op(c, b)
+    x.sum().backward()
+    with torch.no_grad():
+        moved = -eta * c / (1.0 + eta * lam)
+        want = moved.clamp(0.0, 5.0)
+        assert torch.all((x - want).abs() <= 1e-12)
+        assert torch.all((y - eta * (1.0 - 2.0 * want)).abs() <= 1e-12)
+        inside = (moved > 0.0) & (moved < 5.0)
+        assert torch.all((c.grad + inside.double() * (eta / (1.0 + eta * lam))).abs() <= 1e-12)
+    del op, c, x, y, moved, want, inside
+    torch.cuda.empty_cache()
