@@ -16,7 +16,8 @@
 namespace cuopt_amd {
 
 struct hip_error : std::runtime_error {
-  using std::runtime_error::runtime_error;
+  hip_error(const std::string& what, hipError_t c) : std::runtime_error(what), code(c) {}
+  hipError_t code;
 };
 
 #define CUOPT_HIP_CHECK(expr)                                                               \
@@ -25,7 +26,7 @@ struct hip_error : std::runtime_error {
     if (_e != hipSuccess) {                                                                 \
       throw ::cuopt_amd::hip_error(std::string("HIP error '") + hipGetErrorString(_e) +      \
                                    "' at " + __FILE__ + ":" + std::to_string(__LINE__) +    \
-                                   " in " #expr);                                           \
+                                   " in " #expr, _e);                                       \
     }                                                                                       \
   } while (0)
 

@@ -108,7 +108,8 @@ class PoolStore {
   long solves_ = 0;
 };
 
-// hipMalloc, tried again with an emptied store if it fails.
+// hipMalloc, tried again with an emptied store if it fails.  A failure is returned, not left
+// for the next hipGetLastError: the caller may go on with less.
 inline hipError_t pool_malloc(void** p, size_t bytes)
 {
   hipError_t e = hipMalloc(p, bytes);
@@ -116,6 +117,7 @@ inline hipError_t pool_malloc(void** p, size_t bytes)
     (void)hipGetLastError();
     PoolStore::get().trim();
     e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
   }
   return e;
 }

@@ -21,7 +21,8 @@
 // Layout: the caller's vectors are batch-interleaved (v[i * B + b]); the working ones
 // are cut into slabs of W batch members, v[(s * rows + i) * W + w] for member
 // s * W + w, so that the rows of one slab's operand (64 bytes each for the usual W)
-// fit one XCD's L2.  A launch gives each XCD a contiguous run of (slab, row block)
+// fit one XCD's L2.  The last slab stores only the members that the batch has (slabs_of),
+// with rows of their width.  A launch gives each XCD a contiguous run of (slab, row block)
 // items, so an XCD gathers from one slab or two.
 #include <algorithm>
 #include <cmath>
@@ -53,10 +54,11 @@ constexpr int kUB = 256;              // 4 wavefronts per workgroup
 // Gathers of W contiguous values use the lanes that a wavefront per row leaves idle below
 // 64 members, and a slab's operand is smaller than the whole: at 20 000 x 50 000 and
 // B = 64 in FP32 slabs of 32 cut the dual step's L2 misses from 733 k to 592 k lines.
-template <int LW_, int VW_>
+template <int LW_, int VW_, bool BIG_>
 struct Lanes {
   static constexpr int LW = LW_;             // lanes per row
   static constexpr int VW = VW_;             // members per lane
+  static constexpr bool BIG = BIG_;          // 64-bit gather offsets
   static constexpr int W  = LW_ * VW_;       // members per slab
   static constexpr int rows_per_wg = kUB / LW_;
 };
@@ -72,9 +74,9 @@ inline int slab_width(Shape s)
 // The shape of a call.  Up to 4 members: 8 lanes to a row up to kFewRows rows and columns,
 // where a row's chain of loads sets the time and eight lanes read it in fewer rounds, and 4
 // lanes above.  207 steps with gradients in FP64, ms, by shape 4x1 / 8x1 (and the kernel
-// of one row per wavefront): 1 104 x 2 760, B 1 5.04 / 4.87 (4.96); 2 000 x 5 000, B 2 5.53 / 5.07
-// (5.55); 5 500 x 13 750, B 4 6.13 / 5.95 (9.86); 8 000 x 20 000, B 1 6.46 / 6.64 (12.3).  Only the
-// smallest lost to one row per wavefront (200 x 500, B 1 4.62 in either against 4.43).
+// of one row per wavefront): 200 x 500, B 1 4.33 / 4.16 (4.40); 1 104 x 2 760, B 1 4.62 / 4.23 (4.95);
+// 2 000 x 5 000, B 2 4.87 / 4.45 (5.57); 5 500 x 13 750, B 4 6.09 / 5.46 (9.84); 8 000 x 20 000, B 1
+// 5.31 / 5.11 (12.2); 12 000 x 30 000, B 1 5.57 / 5.91 (16.5); 20 000 x 50 000, B 1 7.19 / 7.67 (24.9).
 // More members: the least
 // (members computed, those past B included) x (cost per member) among the shapes that
 // leave at least kMinWaves wavefronts (one member per lane always may).  Measured, ms,
@@ -87,7 +89,7 @@ inline int slab_width(Shape s)
 //   FP64 16 000 x 40 000, B 12, 200 steps with gradients    12.9 / 12.5 / 11.2        (21.3)
 //   FP64  5 000 x 12 500, B 24, 200 steps with gradients    7.61 / 9.69 / 8.59        (10.6)
 constexpr long long kMinWaves = 1200;
-constexpr int kFewRows        = 16384;
+constexpr int kFewRows        = 24576;
 
 template <typename V>
 Shape pick_shape(int m, int n, int B)
@@ -120,19 +122,34 @@ Shape pick_shape(int m, int n, int B)
   return best;
 }
 
+// Whether a gather's offset takes 64 bits.  Otherwise it is one 24-bit multiply-add, of the
+// row's number and the bytes that a slab stores of a row.
+template <typename V>
+bool big_offsets(Shape s, int m, int n)
+{
+  const unsigned long long rows = std::max(m, n);
+  return rows >= (1ULL << 24) || rows * slab_width(s) * sizeof(V) >= (1ULL << 32);
+}
+
 // Calls f(Lanes<...>{}) for a shape.
-template <typename V, class F>
-void with_shape(Shape s, F&& f)
+template <typename V, bool BIG, class F>
+void with_lanes(Shape s, F&& f)
 {
   switch (s) {
-    case Shape::k8x1: f(Lanes<8, 1>{}); break;
-    case Shape::k16x1: f(Lanes<16, 1>{}); break;
-    case Shape::k8x2: f(Lanes<8, 2>{}); break;
+    case Shape::k8x1: f(Lanes<8, 1, BIG>{}); break;
+    case Shape::k16x1: f(Lanes<16, 1, BIG>{}); break;
+    case Shape::k8x2: f(Lanes<8, 2, BIG>{}); break;
     case Shape::k8x4:
-      if constexpr (sizeof(V) == 4) f(Lanes<8, 4>{});
+      if constexpr (sizeof(V) == 4) f(Lanes<8, 4, BIG>{});
       break;
-    default: f(Lanes<4, 1>{});
+    default: f(Lanes<4, 1, BIG>{});
   }
+}
+template <typename V, class F>
+void with_shape(Shape s, int m, int n, F&& f)
+{
+  if (big_offsets<V>(s, m, n)) with_lanes<V, true>(s, f);
+  else with_lanes<V, false>(s, f);
 }
 
 // One matrix as the SpMM kernels take it.  runs: in the order in which consecutive
@@ -146,31 +163,56 @@ struct MatView {
   int rows;
 };
 
+// How a batch lies in slabs: `count` of them, and of the last one only the first `last`
+// members of each row are stored.
+struct Slabs {
+  int count, last;
+  __host__ __device__ size_t members(int W) const { return (size_t)(count - 1) * W + last; }
+};
+
 // The kXcds XCDs take the workgroups of a launch in turn.  They lie in rows of at most
 // 2^kGridShift: a row of 2^24 would have 2^32 lanes, more than a launch can count.
-constexpr int kXcds      = 8;
+constexpr unsigned kXcds = 8;
 constexpr int kGridShift = 20;
 
-template <class L>
-dim3 slab_grid(int rows, int slabs)
+// The slabs of B members.  Up to four are stored as they are (VW of a lane together), more
+// in fours: 100 steps with gradients, ms, with the last slab stored whole / exactly / in fours:
+//   FP64 20 000 x 50 000, B 1   4.80 / 3.56 / 3.56      B 33  14.9 / 13.5 / 13.5     B 13  6.76 / 7.53 / 6.75
+//   FP32  2 000 x  5 000, B 1   2.51 / 2.20 / 2.20      B 9   2.61 / 2.80 / 2.60     B 13  2.60 / 2.83 / 2.60
+//   FP32    500 x  1 250, B 5   2.33 / 2.44 / 2.33
+// (rows that start anywhere in a 64-byte line take more requests).  exact: no member more than B,
+// for a shape of one member per lane.
+inline Slabs slabs_of(Shape shape, int B, bool exact = false)
 {
-  const long long items = (long long)((std::max(rows, 1) + L::rows_per_wg - 1) / L::rows_per_wg) * slabs;
+  const int W = slab_width(shape), VW = shape == Shape::k8x4 ? 4 : shape == Shape::k8x2 ? 2 : 1;
+  const int count = (B + W - 1) / W, last = B - (count - 1) * W;
+  const int unit = exact || last <= 4 ? VW : 4;
+  return {count, (last + unit - 1) / unit * unit};
+}
+
+template <class L>
+dim3 slab_grid(int rows, Slabs S)
+{
+  const long long items = (long long)((std::max(rows, 1) + L::rows_per_wg - 1) / L::rows_per_wg) * S.count;
   const long long all = (items + kXcds - 1) / kXcds * kXcds, row = 1LL << kGridShift;
   return dim3((unsigned)std::min(all, row), (unsigned)((all + row - 1) / row));
 }
 
-// This lane's slab, row and first member within the slab; false past the end.
+// This lane's slab, row and first member within the slab; false past the end.  width:
+// the slab's stored members of a row (the same in every lane).  Lanes past it compute
+// member 0 again, since their group hands the row's entries round, and store nothing.
 struct Place {
-  int slab, row, w, k0, k1;
+  int slab, row, w, k0, k1, width;
+  bool live;
 };
 template <class L>
-__device__ inline bool my_place(int rows, int slabs, const int4* __restrict__ runs, Place& p)
+__device__ inline bool my_place(int rows, Slabs S, const int4* __restrict__ runs, Place& p)
 {
   const int blocks = (rows + L::rows_per_wg - 1) / L::rows_per_wg;
-  const int items = blocks * slabs, per = (items + kXcds - 1) / kXcds;
-  const int at   = (int)(blockIdx.y << kGridShift) + (int)blockIdx.x;
-  const int item = at % kXcds * per + at / kXcds;
-  if (at / kXcds >= per || item >= items) return false;
+  const int items = blocks * S.count, per = (items + (int)kXcds - 1) / (int)kXcds;
+  const unsigned at = (blockIdx.y << kGridShift) + blockIdx.x;
+  const int item    = (int)(at % kXcds) * per + (int)(at / kXcds);
+  if ((int)(at / kXcds) >= per || item >= items) return false;
   p.slab        = item / blocks;
   const int pos = (item - p.slab * blocks) * L::rows_per_wg + (int)threadIdx.x / L::LW;
   if (pos >= rows) return false;
@@ -178,14 +220,31 @@ __device__ inline bool my_place(int rows, int slabs, const int4* __restrict__ ru
   p.row = run.x;
   p.k0  = run.y;
   p.k1  = run.z;
-  p.w   = ((int)threadIdx.x % L::LW) * L::VW;
+  p.width = p.slab + 1 == S.count ? S.last : L::W;
+  p.w     = ((int)threadIdx.x % L::LW) * L::VW;
+  p.live  = p.w < p.width;
+  if (!p.live) p.w = 0;
   return true;
 }
 // Offset of the lane's members of row i in a slab array of `rows` rows.
 template <class L>
 __device__ inline size_t slab_at(const Place& p, int rows, int i)
 {
-  return ((size_t)p.slab * rows + i) * L::W + p.w;
+  const size_t slab = (size_t)p.slab * rows * L::W;
+  if constexpr (L::BIG) return slab + (size_t)i * p.width + p.w;
+  return slab + (__umul24(i, p.width) + p.w);
+}
+// Slab, row and member within the slab of element o of a slab array of `rows` rows.
+struct SlabElement {
+  int slab, row, w;
+};
+__device__ inline SlabElement slab_element(size_t o, int rows, int W, Slabs S)
+{
+  const size_t per = (size_t)rows * W;
+  const int slab   = (int)min(o / per, (size_t)(S.count - 1));
+  const size_t r   = o - slab * per;
+  const int width  = slab + 1 == S.count ? S.last : W;
+  return {slab, (int)(r / width), (int)(r % width)};
 }
 
 // VW contiguous values, loaded and stored as one vector.
@@ -247,12 +306,12 @@ __device__ inline void row_dot_chunks(const MatView<V>& M, const Place& p, const
                                       typename AccFor<V>::type (&a)[L::VW], std::integer_sequence<int, I...>)
 {
   using Acc       = typename AccFor<V>::type;
-  using Off       = typename std::conditional<L::W == 4, size_t, unsigned>::type;
   constexpr int C = L::LW, N = L::LW == 4 ? 2 : 1;  // nonzeros per load, loads per chunk
   const int gl    = (int)threadIdx.x % L::LW;
   const int ke    = p.k1;
   const char* base = reinterpret_cast<const char*>(slab);
   const unsigned w = (unsigned)p.w * (unsigned)sizeof(V);
+  const unsigned row = (unsigned)p.width * (unsigned)sizeof(V);
 #pragma unroll
   for (int i = 0; i < L::VW; ++i) a[i] = Acc::zero();
   int ci[N];
@@ -274,8 +333,10 @@ __device__ inline void row_dot_chunks(const MatView<V>& M, const Place& p, const
     Pack<V, L::VW> x[N][C];
     V v[N];
     auto gather = [&](int col) {
-      const Off off = (Off)(unsigned)col * (Off)(L::W * sizeof(V)) + w;
-      return load_pack<V, L::VW>(reinterpret_cast<const V*>(base + off));
+      if constexpr (L::BIG)
+        return load_pack<V, L::VW>(reinterpret_cast<const V*>(base + ((size_t)(unsigned)col * row + w)));
+      else
+        return load_pack<V, L::VW>(reinterpret_cast<const V*>(base + (__umul24((unsigned)col, row) + w)));
     };
 #pragma unroll
     for (int q = 0; q < N; ++q) {
@@ -321,7 +382,7 @@ __device__ inline Pack<V, L::VW> row_bound(const V* __restrict__ b, bool per_mem
 // ---- forward ----------------------------------------------------------------
 
 template <typename V, class L>
-__global__ __launch_bounds__(kUB) void unr_primal(MatView<V> T, int m, int slabs, const V* __restrict__ y,
+__global__ __launch_bounds__(kUB) void unr_primal(MatView<V> T, int m, Slabs slabs, const V* __restrict__ y,
                                                   const V* __restrict__ x, const V* __restrict__ c,
                                                   const V* __restrict__ lb, const V* __restrict__ ub, V tau,
                                                   V inv_prox, V* __restrict__ xn, V* __restrict__ xb)
@@ -342,12 +403,13 @@ __global__ __launch_bounds__(kUB) void unr_primal(MatView<V> T, int m, int slabs
     xnew.v[i] = mx(mn(v, hi), lo);
     bar.v[i]  = V(2) * xnew.v[i] - xr.v[i];
   }
+  if (!p.live) return;
   store_pack<V, L::VW>(xn + o, xnew);
   store_pack<V, L::VW>(xb + o, bar);
 }
 
 template <typename V, class L>
-__global__ __launch_bounds__(kUB) void unr_dual(MatView<V> A, int n, int slabs, const V* __restrict__ xb,
+__global__ __launch_bounds__(kUB) void unr_dual(MatView<V> A, int n, Slabs slabs, const V* __restrict__ xb,
                                                 const V* __restrict__ y, const V* __restrict__ lc,
                                                 const V* __restrict__ uc, int ldb, V sigma, V* __restrict__ yn)
 {
@@ -365,6 +427,7 @@ __global__ __launch_bounds__(kUB) void unr_dual(MatView<V> A, int n, int slabs, 
     const V proj = mx(-hi.v[i], mn(t, -lo.v[i]));
     out.v[i]     = (t - proj) * sigma;
   }
+  if (!p.live) return;
   store_pack<V, L::VW>(yn + o, out);
 }
 
@@ -415,9 +478,9 @@ __global__ __launch_bounds__(kUB) void unr_flush(size_t n, float* __restrict__ p
 }
 
 // Start of the reverse sweep: gt for the last step from the upstream y-gradient
-// (tot = m W slabs elements of slab arrays).
+// (tot elements of slab arrays).
 template <typename V>
-__global__ __launch_bounds__(kUB) void unr_adj_start(size_t tot, int m, int W, const V* ay,  // may alias gt
+__global__ __launch_bounds__(kUB) void unr_adj_start(size_t tot, int m, int W, Slabs S, const V* ay,  // may alias gt
                                                      const V* __restrict__ yplus, const V* __restrict__ lc,
                                                      const V* __restrict__ uc, int ldb, V sigma, V* gt,
                                                      typename GradAcc<V>::type* __restrict__ glc,
@@ -425,7 +488,7 @@ __global__ __launch_bounds__(kUB) void unr_adj_start(size_t tot, int m, int W, c
 {
   using GA = typename GradAcc<V>::type;
   for (size_t o = blockIdx.x * (size_t)kUB + threadIdx.x; o < tot; o += (size_t)gridDim.x * kUB) {
-    const size_t q = ldb ? o : (o / W) % m;  // per-member bounds, or one per row
+    const size_t q = ldb ? o : slab_element(o, m, W, S).row;  // per-member bounds, or one per row
     double dl, du;
     gt[o] = dual_adjoint(ay ? ay[o] : V(0), yplus[o], lc[q], uc[q], sigma, dl, du);
     glc[o] += (GA)dl;
@@ -436,7 +499,7 @@ __global__ __launch_bounds__(kUB) void unr_adj_start(size_t tot, int m, int W, c
 // Rows j of A^T: gxb = -A^T gt; gw = inner(x+) (ax + 2 gxb) / (1 + tau lam);
 // ax <- gw - gxb (adjoint of x before the step); gc_acc += gw (FP64).
 template <typename V, class L>
-__global__ __launch_bounds__(kUB) void unr_adj_primal(MatView<V> T, int m, int slabs, const V* __restrict__ gt,
+__global__ __launch_bounds__(kUB) void unr_adj_primal(MatView<V> T, int m, Slabs slabs, const V* __restrict__ gt,
                                                       const V* __restrict__ xplus, const V* __restrict__ lb,
                                                       const V* __restrict__ ub, V inv_prox, V* __restrict__ ax,
                                                       V* __restrict__ gw,
@@ -460,6 +523,7 @@ __global__ __launch_bounds__(kUB) void unr_adj_primal(MatView<V> T, int m, int s
     an.v[i]     = w.v[i] - gxb;
     gc.v[i]     = gc.v[i] + (GA)w.v[i];
   }
+  if (!p.live) return;
   store_pack<V, L::VW>(gw + o, w);
   store_pack<V, L::VW>(ax + o, an);
   store_pack<GA, L::VW>(gc_acc + o, gc);
@@ -469,7 +533,7 @@ __global__ __launch_bounds__(kUB) void unr_adj_primal(MatView<V> T, int m, int s
 // step, its gt from ay_prev and the clamp states of its y+ (= y before this step).
 // gt is read and rewritten in place, element by element.
 template <typename V, class L>
-__global__ __launch_bounds__(kUB) void unr_adj_dual(MatView<V> A, int n, int slabs, const V* __restrict__ gw, V tau,
+__global__ __launch_bounds__(kUB) void unr_adj_dual(MatView<V> A, int n, Slabs slabs, const V* __restrict__ gw, V tau,
                                                     V sigma, const V* __restrict__ yprev, const V* __restrict__ lc,
                                                     const V* __restrict__ uc, int ldb, V* __restrict__ gt,
                                                     typename GradAcc<V>::type* __restrict__ glc,
@@ -494,21 +558,22 @@ __global__ __launch_bounds__(kUB) void unr_adj_dual(MatView<V> A, int n, int sla
     glo.v[i] = glo.v[i] + (GA)dl;
     guo.v[i] = guo.v[i] + (GA)du;
   }
+  if (!p.live) return;
   store_pack<V, L::VW>(gt + o, gto);
   store_pack<GA, L::VW>(glc + o, glo);
   store_pack<GA, L::VW>(guc + o, guo);
 }
 
-// Caller's layout (i * B + b) to slabs of W members; members past B are zero.
+// Caller's layout (i * B + b) to slabs of W members; stored members past B are zero.
 template <typename V>
-__global__ __launch_bounds__(kUB) void unr_convert_in(int rows, int B, int W, int slabs, const double* __restrict__ in,
+__global__ __launch_bounds__(kUB) void unr_convert_in(int rows, int B, int W, Slabs S, const double* __restrict__ in,
                                                       V* __restrict__ out)
 {
-  const size_t tot = (size_t)rows * W * slabs;
+  const size_t tot = rows * S.members(W);
   for (size_t o = blockIdx.x * (size_t)kUB + threadIdx.x; o < tot; o += (size_t)gridDim.x * kUB) {
-    const size_t r = o / W;
-    const int s = (int)(r / rows), i = (int)(r - (size_t)s * rows), b = s * W + (int)(o % W);
-    out[o] = b < B ? (V)in[(size_t)i * B + b] : V(0);
+    const SlabElement e = slab_element(o, rows, W, S);
+    const int b         = e.slab * W + e.w;
+    out[o] = b < B ? (V)in[(size_t)e.row * B + b] : V(0);
   }
 }
 template <typename V>
@@ -518,22 +583,22 @@ __global__ __launch_bounds__(kUB) void unr_convert_rows(int rows, const double* 
 }
 // Slabs to the caller's layout, scaled.
 template <typename V>
-__global__ __launch_bounds__(kUB) void unr_convert_out(int rows, int B, int W, const V* __restrict__ in, double scale,
+__global__ __launch_bounds__(kUB) void unr_convert_out(int rows, int B, int W, Slabs S, const V* __restrict__ in, double scale,
                                                        double* __restrict__ out)
 {
   const size_t tot = (size_t)rows * B;
   for (size_t o = blockIdx.x * (size_t)kUB + threadIdx.x; o < tot; o += (size_t)gridDim.x * kUB) {
     const size_t i = o / B;
-    const int b    = (int)(o - i * B);
-    out[o]         = scale * (double)in[((size_t)(b / W) * rows + i) * W + b % W];
+    const int b = (int)(o - i * B), s = b / W;
+    out[o] = scale * (double)in[(size_t)s * rows * W + i * (s + 1 == S.count ? S.last : W) + b % W];
   }
 }
 template <typename V>
-__global__ __launch_bounds__(kUB) void unr_init_x(size_t tot, int n, int W, const V* __restrict__ lb,
+__global__ __launch_bounds__(kUB) void unr_init_x(size_t tot, int n, int W, Slabs S, const V* __restrict__ lb,
                                                   const V* __restrict__ ub, V* __restrict__ x)
 {
   for (size_t o = blockIdx.x * (size_t)kUB + threadIdx.x; o < tot; o += (size_t)gridDim.x * kUB) {
-    const int j = (int)((o / W) % n);
+    const int j = slab_element(o, n, W, S).row;
     x[o]        = mn(mx(V(0), lb[j]), ub[j]);
   }
 }
@@ -573,7 +638,7 @@ __global__ __launch_bounds__(kUB) void unr_spmv64(const int* __restrict__ ptr, c
 
 // Y = A X over slabs (the SpMM timed by the batch-size search).
 template <typename V, class L>
-__global__ __launch_bounds__(kUB) void unr_spmm(MatView<V> M, int cols, int slabs, const V* __restrict__ x,
+__global__ __launch_bounds__(kUB) void unr_spmm(MatView<V> M, int cols, Slabs slabs, const V* __restrict__ x,
                                                 V* __restrict__ y)
 {
   Place p;
@@ -583,6 +648,7 @@ __global__ __launch_bounds__(kUB) void unr_spmm(MatView<V> M, int cols, int slab
   Pack<V, L::VW> out;
 #pragma unroll
   for (int i = 0; i < L::VW; ++i) out.v[i] = s[i].value();
+  if (!p.live) return;
   store_pack<V, L::VW>(y + slab_at<L>(p, M.rows, p.row), out);
 }
 
@@ -625,7 +691,8 @@ struct UnrolledImpl {
   bool ready = false;
   int B = 0, K = 0, every = 1, ldb = 0;
   Shape shape = Shape::k4x1;
-  int W = 4, slabs = 0;  // members per slab, slabs
+  int W = 4;  // members per slab
+  Slabs slabs{0, 0};
   DevBuf<unsigned char> work;  // typed views below
   size_t ckpt_off = 0, seg_off = 0;
   DevBuf<int> seg;  // checkpoint segment counter read by the segment graphs
@@ -719,7 +786,7 @@ struct Work {
 template <typename V>
 Work<V> carve(UnrolledImpl& U, int nseg, bool allocate)
 {
-  const size_t members = (size_t)U.W * U.slabs;
+  const size_t members = U.slabs.members(U.W);
   const size_t nB = U.n * members, mB = U.m * members, lcn = U.ldb ? mB : (size_t)U.m;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -755,7 +822,7 @@ template <typename V>
 void step(const Views<V>& M, UnrolledImpl& U, const Work<V>& W, const V* x, const V* y, V* xn, V* yn, hipStream_t s)
 {
   const V tau = (V)U.eta, sigma = (V)U.eta, inv_prox = (V)(1.0 / (1.0 + U.eta * U.lam));
-  with_shape<V>(U.shape, [&](auto lanes) {
+  with_shape<V>(U.shape, U.m, U.n, [&](auto lanes) {
     using L = decltype(lanes);
     hipLaunchKernelGGL((unr_primal<V, L>), slab_grid<L>(U.n, U.slabs), dim3(kUB), 0, s, M.T, U.m, U.slabs, y, x,
                        (const V*)W.c, M.lb, M.ub, tau, inv_prox, xn, W.xb);
@@ -771,12 +838,12 @@ void forward_impl(UnrolledImpl& U, const double* c, const double* lc, const doub
   const int nseg = (U.K + U.every - 1) / U.every;
   Work<V> W      = carve<V>(U, nseg, true);
   Views<V> M     = views<V>(U);
-  const size_t members = (size_t)U.W * U.slabs, nB = U.n * members, mB = U.m * members;
+  const size_t members = U.slabs.members(U.W), nB = U.n * members, mB = U.m * members;
   if (!U.seg.get()) U.seg.resize(1);
-  // The captured graphs hold the work buffer's addresses and the shapes.  Where carve()
+  // The captured graphs hold the work buffer's addresses and the layout.  Where carve()
   // places the checkpoints and all that follows them goes by the number of segments.
   const std::vector<long long> key{(long long)(uintptr_t)U.work.get(), U.B, nseg, U.every, U.ldb,
-                                   (long long)sizeof(V), (long long)U.shape};
+                                   (long long)sizeof(V), (long long)U.shape, U.slabs.last};
   if (key != U.graph_key) {
     U.drop_graphs();
     U.graph_key = key;
@@ -788,7 +855,7 @@ void forward_impl(UnrolledImpl& U, const double* c, const double* lc, const doub
     else
       hipLaunchKernelGGL(unr_convert_rows<V>, dim3(ew_blocks(U.m)), dim3(kUB), 0, s, U.m, from, to);
   }
-  hipLaunchKernelGGL(unr_init_x<V>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, nB, U.n, U.W, M.lb, M.ub, W.x[0]);
+  hipLaunchKernelGGL(unr_init_x<V>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, nB, U.n, U.W, U.slabs, M.lb, M.ub, W.x[0]);
   hipLaunchKernelGGL(unr_zero<V>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, mB, W.y[0]);
   hipLaunchKernelGGL(unr_seg_update, dim3(1), dim3(kWave), 0, s, U.seg.get(), 0, 1);
   // One segment from buffer p: checkpoint (x, y) into slot *seg, advance the
@@ -815,11 +882,11 @@ void forward_impl(UnrolledImpl& U, const double* c, const double* lc, const doub
     cur ^= (L & 1);
   }
   CUOPT_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(unr_convert_out<V>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, U.n, U.B, U.W, (const V*)W.x[cur], 1.0,
+  hipLaunchKernelGGL(unr_convert_out<V>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, U.n, U.B, U.W, U.slabs, (const V*)W.x[cur], 1.0,
                      x_out);
   if (y_out)
-    hipLaunchKernelGGL(unr_convert_out<V>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, U.m, U.B, U.W, (const V*)W.y[cur],
-                       1.0, y_out);
+    hipLaunchKernelGGL(unr_convert_out<V>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, U.m, U.B, U.W, U.slabs,
+                       (const V*)W.y[cur], 1.0, y_out);
   // final state kept for the backward pass (segment states are recomputed)
   CUOPT_HIP_CHECK(hipGetLastError());
 }
@@ -831,7 +898,7 @@ void backward_impl(UnrolledImpl& U, const double* gx, const double* gy, double* 
   const int nseg  = (U.K + U.every - 1) / U.every;
   Work<V> W       = carve<V>(U, nseg, false);
   Views<V> M      = views<V>(U);
-  const size_t members = (size_t)U.W * U.slabs, nB = U.n * members, mB = U.m * members;
+  const size_t members = U.slabs.members(U.W), nB = U.n * members, mB = U.m * members;
   const V tau = (V)U.eta, sigma = (V)U.eta, inv_prox = (V)(1.0 / (1.0 + U.eta * U.lam));
   hipLaunchKernelGGL(unr_zero64, dim3(ew_blocks(nB)), dim3(kUB), 0, s, nB, W.gc);
   hipLaunchKernelGGL(unr_zero64, dim3(ew_blocks(mB)), dim3(kUB), 0, s, mB, W.glc);
@@ -865,10 +932,10 @@ void backward_impl(UnrolledImpl& U, const double* gx, const double* gy, double* 
       const V* xplus = W.sx + (size_t)(t + 1) * nB;
       const V* yplus = W.sy + (size_t)(t + 1) * mB;
       if (last && t == L - 1)
-        hipLaunchKernelGGL(unr_adj_start<V>, dim3(ew_blocks(mB)), dim3(kUB), 0, q, mB, U.m, U.W,
+        hipLaunchKernelGGL(unr_adj_start<V>, dim3(ew_blocks(mB)), dim3(kUB), 0, q, mB, U.m, U.W, U.slabs,
                            gy ? (const V*)W.gt : (const V*)nullptr, yplus, (const V*)W.lc, (const V*)W.uc, U.ldb,
                            sigma, W.gt, W.plc, W.puc);
-      with_shape<V>(U.shape, [&](auto lanes) {
+      with_shape<V>(U.shape, U.m, U.n, [&](auto lanes) {
         using L = decltype(lanes);
         hipLaunchKernelGGL((unr_adj_primal<V, L>), slab_grid<L>(U.n, U.slabs), dim3(kUB), 0, q, M.T, U.m, U.slabs,
                            (const V*)W.gt, xplus, M.lb, M.ub, inv_prox, W.ax, W.gw, W.pc);
@@ -898,11 +965,11 @@ void backward_impl(UnrolledImpl& U, const double* gx, const double* gy, double* 
   }
   CUOPT_HIP_CHECK(hipGetLastError());
   // gc = -tau / (1 + tau lam) * sum of gw: the kernel accumulated gw, already divided by (1 + tau lam).
-  hipLaunchKernelGGL(unr_convert_out<double>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, U.n, U.B, U.W,
+  hipLaunchKernelGGL(unr_convert_out<double>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, U.n, U.B, U.W, U.slabs,
                      (const double*)W.gc, -U.eta, gc);
-  hipLaunchKernelGGL(unr_convert_out<double>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, U.m, U.B, U.W,
+  hipLaunchKernelGGL(unr_convert_out<double>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, U.m, U.B, U.W, U.slabs,
                      (const double*)W.glc, 1.0, glc);
-  hipLaunchKernelGGL(unr_convert_out<double>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, U.m, U.B, U.W,
+  hipLaunchKernelGGL(unr_convert_out<double>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, U.m, U.B, U.W, U.slabs,
                      (const double*)W.guc, 1.0, guc);
   CUOPT_HIP_CHECK(hipGetLastError());
 }
@@ -1031,15 +1098,24 @@ void unrolled_forward(UnrolledHandle* h, int B, int K, int every, const double* 
   U->K     = K;
   U->every = every;
   U->ldb   = bounds_per_batch ? B : 0;
-  U->shape = U->precision == CUOPT_AMD_PRECISION_FP32_MIXED ? pick_shape<float>(U->m, U->n, B)
-                                                            : pick_shape<double>(U->m, U->n, B);
-  U->W     = slab_width(U->shape);
-  U->slabs = (B + U->W - 1) / U->W;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (U->precision == CUOPT_AMD_PRECISION_FP32_MIXED)
-    forward_impl<float>(*U, c, lc, uc, x, y, s);
-  else
-    forward_impl<double>(*U, c, lc, uc, x, y, s);
+  const bool fp32 = U->precision == CUOPT_AMD_PRECISION_FP32_MIXED;
+  hipStream_t s   = static_cast<hipStream_t>(stream);
+  auto run = [&](Shape shape, bool exact) {
+    U->shape = shape;
+    U->W     = slab_width(shape);
+    U->slabs = slabs_of(shape, B, exact);
+    if (fp32) forward_impl<float>(*U, c, lc, uc, x, y, s);
+    else forward_impl<double>(*U, c, lc, uc, x, y, s);
+  };
+  const Shape shape = fp32 ? pick_shape<float>(U->m, U->n, B) : pick_shape<double>(U->m, U->n, B);
+  try {
+    run(shape, false);
+  } catch (const hip_error& e) {
+    // Where the stored members past B do not fit, B alone may.
+    const Shape narrow = shape == Shape::k8x2 || shape == Shape::k8x4 ? Shape::k16x1 : shape;
+    if (e.code != hipErrorOutOfMemory || U->slabs.members(U->W) == (size_t)B) throw;
+    run(narrow, true);
+  }
   U->ready = true;
 }
 
@@ -1080,14 +1156,15 @@ int optimal_batch_size_impl(UnrolledImpl& U, int max_batch)
     CUOPT_HIP_CHECK(hipEventCreate(&e1));
     auto cost = [&](int B) {
       const Shape shape = pick_shape<V>(U.m, U.n, B);
-      const int W = slab_width(shape), slabs = (B + W - 1) / W;
-      const size_t nB = (size_t)std::max(U.n, 1) * W * slabs, mB = (size_t)std::max(U.m, 1) * W * slabs;
+      const Slabs slabs    = slabs_of(shape, B);
+      const size_t members = slabs.members(slab_width(shape)), nB = std::max(U.n, 1) * members,
+                   mB = std::max(U.m, 1) * members;
       if (x.size() < nB) x.resize(nB);
       if (y.size() < mB) y.resize(mB);
       hipLaunchKernelGGL(unr_zero<V>, dim3(ew_blocks(nB)), dim3(kUB), 0, s, nB, x.get());
       hipLaunchKernelGGL(unr_zero<V>, dim3(ew_blocks(mB)), dim3(kUB), 0, s, mB, y.get());
       auto run = [&]() {
-        with_shape<V>(shape, [&](auto lanes) {
+        with_shape<V>(shape, U.m, U.n, [&](auto lanes) {
           using L = decltype(lanes);
           if (U.m > 0)
             hipLaunchKernelGGL((unr_spmm<V, L>), slab_grid<L>(U.m, slabs), dim3(kUB), 0, s, M.A, U.n, slabs,

@@ -418,3 +418,91 @@ def test_more_workgroups_than_one_grid_dimension_counts():
         assert torch.all((c.grad + inside.double() * (eta / (1.0 + eta * lam))).abs() <= 1e-12)
     del op, c, x, y, moved, want, inside
     torch.cuda.empty_cache()
+
+
+def test_working_storage_needs_no_more_than_the_batch(monkeypatch):
+    # Slabs hold more members than a batch that their width does not divide.  Where only
+    # the batch itself fits the memory that is left, the call still runs, with the same
+    # result: the segment states of `every` steps are most of the storage here, 6 GB of
+    # 7 GB left free, which whole slabs of this many members would pass.
+    lp, _ = ragged_lp(seed=8, m=300, n=700)
+    rng = np.random.default_rng(8)
+
+    def run(prec, B, shape, every):
+        print(f"working storage {prec} B={B} shape={shape} every={every}", flush=True)
+        if shape:
+            monkeypatch.setenv("CUOPT_AMD_UNR_SHAPE", str(shape))
+        else:
+            monkeypatch.delenv("CUOPT_AMD_UNR_SHAPE", raising=False)
+        op = UnrolledPDHG(lp, ridge=1e-3, steps=12, checkpoint_every=every, precision=prec)
+        c, b = (torch.tensor(v, device=DEV, requires_grad=True) for v in (c0[:B], lp.con_lb))
+        x, y = op(c, b)
+        torch.autograd.backward([x, y], [gx[:B], torch.ones_like(y)])
+        return [v.detach().cpu().numpy() for v in (x, y, c.grad, b.grad)]
+
+    cases = [("fp64", 1, None), ("fp64", 5, None), ("fp64", 9, 82), ("fp32_mixed", 3, None), ("fp32_mixed", 9, None),
+             ("fp32_mixed", 37, 84)]
+    c0 = lp.c[None, :] + 0.1 * rng.normal(size=(37, lp.n))
+    gx = torch.tensor(rng.normal(size=(37, lp.n)), device=DEV)
+    want = [run(*case, 12) for case in cases]
+    torch.cuda.empty_cache()
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - (7 << 30), dtype=torch.uint8, device=DEV)
+    try:
+        got = [run(*case, (6 << 30) // ((8 if case[0] == "fp64" else 4) * case[1] * (lp.m + lp.n))) for case in cases]
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    for case, a, b in zip(cases, want, got):
+        for name, u, v in zip(("x", "y", "gc", "gb"), a, b):
+            assert np.array_equal(u, v), (case, name)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_more_columns_than_24_bits_number(monkeypatch, prec):
+    # Gathers take a 64-bit offset from 2^24 rows or columns up.  Columns without nonzeros
+    # change nothing for the others, so a matrix whose few nonzeros lie among 2^24 + 40 columns
+    # gives, bit for bit, what the matrix of its nonzero columns does, in every shape.
+    import scipy.sparse as sp
+
+    rng = np.random.default_rng(12)
+    m, n, B = 70, (1 << 24) + 40, 7
+    used = np.unique(np.concatenate([rng.choice(n, size=900, replace=False), np.arange(n - 45, n), np.arange(3)]))
+    small = sp.random(m, used.size, density=0.03, random_state=12, format="csc", data_rvs=rng.standard_normal)
+    small = (small + sp.csc_matrix((np.ones(used.size), (np.arange(used.size) % m, np.arange(used.size))),
+                                   shape=(m, used.size))).tocsr()
+    small.sort_indices()
+    b = small @ rng.random(used.size)
+
+    def lp_of(cols, width):
+        return G.LP(m=m, n=width, row_offsets=small.indptr.astype(np.int32), col_indices=cols.astype(np.int32),
+                    values=small.data, c=np.zeros(width), con_lb=b, con_ub=b.copy(), var_lb=np.zeros(width),
+                    var_ub=np.full(width, 10.0))
+
+    kw = dict(ridge=1e-3, steps=3, checkpoint_every=2, precision=prec)
+    few = UnrolledPDHG(lp_of(small.indices, used.size), **kw)
+    many = UnrolledPDHG(lp_of(used[small.indices], n), **kw)
+    assert few.step_size == many.step_size
+    at = torch.tensor(used, device=DEV)
+    c0 = torch.tensor(rng.normal(size=(B, used.size)), device=DEV)
+    gx = torch.tensor(rng.normal(size=(B, used.size)), device=DEV)
+
+    def run(op, wide):
+        c = c0
+        if wide:
+            c = torch.zeros(B, n, dtype=torch.float64, device=DEV)
+            c[:, at] = c0
+        c = c.clone().requires_grad_(True)
+        bt = torch.tensor(b, device=DEV, requires_grad=True)
+        x, y = op(c, bt)
+        ((x[:, at] if wide else x) * gx).sum().backward()
+        gc = c.grad[:, at] if wide else c.grad
+        return [v.detach().cpu().numpy() for v in (x[:, at] if wide else x, y, gc, bt.grad)]
+
+    want = run(few, False)
+    for shape in (41, 81, 161, 82) + ((84,) if prec == "fp32_mixed" else ()):
+        print(f"2^24 columns {prec} shape {shape}", flush=True)
+        monkeypatch.setenv("CUOPT_AMD_UNR_SHAPE", str(shape))
+        for name, u, v in zip(("x", "y", "gc", "gb"), want, run(many, True)):
+            assert np.array_equal(u, v), (shape, name)
+    del many
+    torch.cuda.empty_cache()
