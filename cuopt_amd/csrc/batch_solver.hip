@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "batch_solver.hpp"
+#include "batch_width.hpp"
 #include "common.hpp"
 #include "pdlp_kernels.hpp"
 
@@ -46,14 +47,13 @@ namespace {
 
 // Lanes per LP workgroup: a narrow workgroup of kRef lanes, two to a CU, or a wide one
 // of kWide lanes with a CU of its own and all of its LDS, so that every gathered
-// vector fits.  One LP takes about 0.55 times as long per iteration when wide (m 1 200 to
+// vector fits.  One LP takes about 0.62 times as long per iteration when wide (m 1 200 to
 // 2 000: FP32-mixed 75.7 -> 47.1 us, FP64 132.6 -> 82.8 us; 512 lanes 48.1 / 86.4 us), but
 // it takes twice the share of the chip.  With few LPs the largest ones set the time of
-// the launch and with many the sum does, so the host picks the width by the
-// estimate of both (prefer_wide): 1 024 LPs of m 50 to 2 000 in FP32-mixed 119 ->
+// the launch and with many the sum does, so the host picks the width by an
+// estimate of the launch (prefer_wide): 1 024 LPs of m 50 to 2 000 in FP32-mixed 119 ->
 // 75 ms, 512 in FP64 188 -> 117 ms with wide ones; 4 096 in FP32-mixed 216 ms narrow
-// against 252 ms.  LPs of fewer than kWideNnz nonzeros are narrow in any batch
-// (9 us per iteration either way).
+// against 252 ms.
 //
 // Every reduction over an LP is summed in the order of kRef lanes (lane v holds the
 // terms v, v + kRef, ... of an elementwise sum, and in a row pass those of the rows
@@ -61,7 +61,6 @@ namespace {
 // an LP's result does not depend on the workgroup that solves it, bit for bit.
 constexpr int kRef     = 256;
 constexpr int kWide    = 768;
-constexpr int kWideNnz = 2000;
 
 // Workgroups per CU that a width is built for (its register budget,
 // __launch_bounds__, and the LDS share of each).  Three narrow ones (at most 168
@@ -1231,27 +1230,12 @@ void host_parallel_for(int count, F f)
   if (err) std::rethrow_exception(err);
 }
 
-// Whether LPs of at least kWideNnz nonzeros get wide workgroups.  The launch takes at
-// least as long as its longest LP, and as the CU time of all of them over the CUs;
-// both are estimated per iteration (the LPs' iteration counts are not known) from
-// the measured 6 + 2.6 z us of a narrow workgroup (half a CU) and 6.5 + 1.3 z us of a
-// wide one, z being the LP's nonzeros in thousands.
-bool prefer_wide(const std::vector<BatchDesc>& desc, const std::vector<int>& active)
+int cu_count()
 {
   int dev = 0, cus = 0;
   CUOPT_HIP_CHECK(hipGetDevice(&dev));
   CUOPT_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  double sum_n = 0.0, max_n = 0.0, sum_w = 0.0, max_w = 0.0;
-  for (int a : active) {
-    const double z  = 1e-3 * desc[a].nnz;
-    const bool w    = desc[a].nnz >= kWideNnz;
-    const double tn = 6.0 + 2.6 * z, tw = w ? 6.5 + 1.3 * z : tn;
-    sum_n += tn / wg_per_cu(kRef);
-    sum_w += tw / (w ? wg_per_cu(kWide) : wg_per_cu(kRef));
-    max_n = std::max(max_n, tn);
-    max_w = std::max(max_w, tw);
-  }
-  return std::max(sum_w / cus, max_w) < std::max(sum_n / cus, max_n);
+  return cus;
 }
 
 template <typename V>
@@ -1326,9 +1310,10 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
       std::copy(ucs[a].begin(), ucs[a].end(), h_uc.get() + d.row0);
     }
   };
-  const bool wide = prefer_wide(desc, active);
-  // row blocks of A and A^T for each LP
+  // row blocks of A and A^T for each LP, narrow (aref, tref) and, where it gains from it, wide
   std::vector<std::vector<int>> ablocks(lps.size()), tblocks(lps.size()), aref(lps.size()), tref(lps.size());
+  auto count = [](const std::vector<int>& blocks) { return (int)blocks.size() - 1; };
+  auto gains = [&](int a) { return gains_from_width(desc[a].nnz, count(aref[a]) + count(tref[a])); };
   {
     auto plan = [&](int t, int nt) {
       std::vector<int> cnt;
@@ -1341,7 +1326,7 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
         for (int k = 0; k < desc[a].nnz; ++k) ++cnt[lp.colidx[k]];
         plan_row_blocks(lp.m, desc[a].lga, kRef, alen, aref[a]);
         plan_row_blocks(lp.n, desc[a].lgt, kRef, tlen, tref[a]);
-        if (wide && desc[a].nnz >= kWideNnz) {
+        if (gains(a)) {
           plan_row_blocks(lp.m, desc[a].lga, kWide, alen, ablocks[a]);
           plan_row_blocks(lp.n, desc[a].lgt, kWide, tlen, tblocks[a]);
         }
@@ -1352,29 +1337,33 @@ std::vector<SolveResult> run_batch(const std::vector<const LpHost*>& lps,
     for (int t = 0; t < nt; ++t) th.emplace_back(plan, t, nt);
     for (auto& t : th) t.join();
   }
+  std::vector<BatchLp> sizes;
+  for (int a : active)
+    sizes.push_back({desc[a].nnz, count(aref[a]) + count(tref[a]), gains(a) ? count(ablocks[a]) + count(tblocks[a]) : 0});
+  const bool wide = prefer_wide(sizes, cu_count(), std::is_same<V, float>::value);
+  auto is_wide    = [&](int a) { return wide && gains(a); };
   std::vector<int> h_blk;
   for (int a : active) {
     BatchDesc& d = desc[a];
-    auto put     = [&](const std::vector<int>& v, int& first, int& count) {
-      first = (int)h_blk.size();
-      count = (int)v.size() - 1;
+    auto put     = [&](const std::vector<int>& v, int& first, int& blocks) {
+      first  = (int)h_blk.size();
+      blocks = count(v);
       h_blk.insert(h_blk.end(), v.begin(), v.end());
     };
     put(aref[a], d.aref0, d.naref);
     put(tref[a], d.tref0, d.ntref);
     d.ablk0 = d.aref0, d.nablk = d.naref;
     d.tblk0 = d.tref0, d.ntblk = d.ntref;
-    if (wide && d.nnz >= kWideNnz) {
+    if (is_wide(a)) {
       put(ablocks[a], d.ablk0, d.nablk);
       put(tblocks[a], d.tblk0, d.ntblk);
     }
   }
 
-  // processing order: largest first
+  // processing order: the wide ones first, largest first
   std::vector<int> order(active);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return desc[x].nnz > desc[y].nnz; });
-  int nwide = 0;  // the first ones, by their order
-  while (wide && nwide < nb && desc[order[nwide]].nnz >= kWideNnz) ++nwide;
+  const int nwide = (int)(std::stable_partition(order.begin(), order.end(), is_wide) - order.begin());
   std::vector<double> z0(std::max(max_m, 1));
   {
     std::mt19937 gen(1);
