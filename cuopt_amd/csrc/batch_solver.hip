@@ -1750,6 +1750,7 @@ std::vector<SolveResult> batch_solve(const std::vector<const LpHost*>& lps, cons
   });
   for (size_t a = 0; a < lps.size(); ++a)
     if (on_device[a]) active.push_back((int)a);
+  PoolStore::get().age();
   // LPs answered on the host above keep their results if the device part fails.
   std::vector<SolveResult> keep = R;
   try {

@@ -10,8 +10,9 @@
 // is on one stream, so the order of the launches orders the uses too.  When the solve
 // ends (its stream is idle) the lease hands its blocks to a process-wide store, which
 // keeps at most kPoolCap bytes, the oldest freed first, and none that the last kPoolAge
-// solves left unused; it is emptied by cuOptAmdReleaseMemory and when an allocation
-// fails.  It outlives the handles: freeing with the last of them would only move the cost
+// solves, batches among them, left unused; it is emptied by cuOptAmdReleaseMemory, when an
+// allocation fails, and when a differentiable operator is made, whose program goes on with
+// other work.  It outlives the handles: freeing with the last of them would only move the cost
 // to a caller that makes its handles anew for each solve.  Contents are never reused:
 // an array from the store is as undefined as one from hipMalloc.
 #pragma once
@@ -90,6 +91,12 @@ class PoolStore {
     }
     pool_free(out);
   }
+  // A batch solve, which takes its memory elsewhere, ages the blocks as a solve does.
+  void age()
+  {
+    std::list<PoolBlock> none;
+    give(none);
+  }
   void trim()
   {
     std::list<PoolBlock> out;
@@ -152,6 +159,7 @@ class PoolLease {
       (void)hipStreamSynchronize(s);
       pool_free(free_);
       e = hipMalloc(&b.p, bytes);
+      if (e != hipSuccess) (void)hipGetLastError();
     }
     if (e != hipSuccess) b = PoolBlock{};
     return e;

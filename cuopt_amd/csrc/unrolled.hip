@@ -996,6 +996,7 @@ UnrolledHandle* unrolled_create(int m, int n, const int* rowptr, const int* coli
                                 const double* lb, const double* ub, double lam, int precision)
 {
   auto* U = new UnrolledImpl();
+  PoolStore::get().trim();
   try {
     U->m = m;
     U->n = n;

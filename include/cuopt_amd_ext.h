@@ -325,7 +325,8 @@ cuopt_int_t cuOptAmdBatchSolve(cuopt_int_t num_problems,
                                cuOptSolution* solutions);
 
 /* Frees the device memory kept from finished solves for the next ones (at most 2 GiB
- * a process).  It is safe at any time, solves on other threads included. */
+ * a process; what eight solves or batches did not use is freed by itself, and all of it
+ * when a handle of the differentiable map is made).  It is safe at any time, solves on other threads included. */
 void cuOptAmdReleaseMemory(void);
 
 #ifdef __cplusplus

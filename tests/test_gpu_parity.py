@@ -970,3 +970,38 @@ def test_memory_kept_between_solves(prec):
             assert np.array_equal(getattr(a, f), getattr(b, f)), f
     c_api.release_memory()
     assert torch.cuda.mem_get_info()[0] >= free - (16 << 20)
+
+
+def test_kept_memory_goes_back_to_a_program_that_does_other_work():
+    # Memory that single solves left is freed when nine batches have not used it, and when
+    # an operator of the differentiable map is made.
+    import torch
+
+    from cuopt_amd.autograd import UnrolledPDHG
+
+    large = c_api.Problem(G.banded_lp(m=100_000, width=8, seed=1))
+    small = [c_api.Problem(G.random_lp(m=20, n=50, seed=i)) for i in range(3)]
+    conf = c_api.make_settings(1e-8, "fp64", 10, 60.0)
+    lp = G.random_lp(m=30, n=80, seed=4)
+
+    def held(work):
+        c_api.release_memory()
+        before = torch.cuda.mem_get_info()[0]
+        c_api.solve_problem(large, conf)
+        kept = before - torch.cuda.mem_get_info()[0]
+        work()
+        return kept, before - torch.cuda.mem_get_info()[0]
+
+    def batches():
+        for _ in range(9):
+            c_api.batch_solve(small, tol=1e-3, iteration_limit=20)
+
+    def operator():
+        keep.append(UnrolledPDHG(lp, ridge=1e-3, steps=4, checkpoint_every=2, precision="fp64"))
+
+    keep = []
+    batches(), operator()  # streams, scratch and module loading happen once
+    for work in (batches, operator):
+        kept, left = held(work)
+        assert kept > (32 << 20), (work.__name__, kept)
+        assert left < (16 << 20), (work.__name__, kept, left)
