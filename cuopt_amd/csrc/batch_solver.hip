@@ -28,6 +28,7 @@
 #include <condition_variable>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <numeric>
 #include <random>
@@ -1751,12 +1752,28 @@ std::vector<SolveResult> batch_solve(const std::vector<const LpHost*>& lps, cons
   for (size_t a = 0; a < lps.size(); ++a)
     if (on_device[a]) active.push_back((int)a);
   PoolStore::get().age();
-  // LPs answered on the host above keep their results if the device part fails.
-  std::vector<SolveResult> keep = R;
+  // LPs answered on the host above keep their results if the device part fails.  A batch
+  // whose working arrays do not fit the device's free memory (52 bytes a nonzero in
+  // FP32-mixed, 44 in FP64, beside its vectors) is solved in halves, one after the other.
+  std::function<void(const std::vector<int>&)> run = [&](const std::vector<int>& part) {
+    try {
+      std::vector<SolveResult> res(lps.size());
+      if (st.precision == CUOPT_AMD_PRECISION_FP32_MIXED)
+        res = run_batch<float>(lps, part, lcs, ucs, st, std::move(res));
+      else
+        res = run_batch<double>(lps, part, lcs, ucs, st, std::move(res));
+      for (int a : part) R[a] = std::move(res[a]);
+      return;
+    } catch (const hip_error& e) {
+      if (e.code != hipErrorOutOfMemory || part.size() < 2) throw;
+    }
+    const auto mid = part.begin() + (part.size() + 1) / 2;
+    run(std::vector<int>(part.begin(), mid));
+    run(std::vector<int>(mid, part.end()));
+  };
   try {
-    if (st.precision == CUOPT_AMD_PRECISION_FP32_MIXED)
-      return run_batch<float>(lps, active, lcs, ucs, st, std::move(R));
-    return run_batch<double>(lps, active, lcs, ucs, st, std::move(R));
+    run(active);
+    return R;
   } catch (const std::exception& e) {
     const std::string msg = e.what();
     int code              = CUOPT_RUNTIME_ERROR;
@@ -1764,11 +1781,12 @@ std::vector<SolveResult> batch_solve(const std::vector<const LpHost*>& lps, cons
     if (dynamic_cast<const std::bad_alloc*>(&e) || msg.find("out of memory") != std::string::npos)
       code = CUOPT_OUT_OF_MEMORY;
     for (int a : active) {
-      keep[a].error         = code;
-      keep[a].error_message = msg;
-      keep[a].status        = CUOPT_TERIMINATION_STATUS_NO_TERMINATION;
+      R[a]               = SolveResult{};
+      R[a].error         = code;
+      R[a].error_message = msg;
+      R[a].status        = CUOPT_TERIMINATION_STATUS_NO_TERMINATION;
     }
-    return keep;
+    return R;
   }
 }
 

@@ -1005,3 +1005,28 @@ def test_kept_memory_goes_back_to_a_program_that_does_other_work():
         kept, left = held(work)
         assert kept > (32 << 20), (work.__name__, kept)
         assert left < (16 << 20), (work.__name__, kept, left)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_batch_larger_than_the_free_memory_is_solved_in_parts(prec):
+    # 2 000 LPs of 40 000 nonzeros take about 6 GB of working arrays.  With 4 GB left they are
+    # solved in halves, each LP with the result it has in one launch, bit for bit.
+    import torch
+
+    few = [c_api.Problem(G.random_lp(m=m, n=5000, seed=m)) for m in (1990, 2000)]
+    many = few * 1000
+    kw = dict(tol=1e-9, precision=prec, iteration_limit=20, time_limit=60.0)
+    want = c_api.batch_solve(few, **kw)
+    c_api.release_memory()
+    torch.cuda.empty_cache()
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - (4 << 30), dtype=torch.uint8, device="cuda")
+    try:
+        got = c_api.batch_solve(many, **kw)
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    for i, r in enumerate(got):
+        w = want[i % 2]
+        assert (r.status, r.iterations) == (w.status, w.iterations), i
+        for f in ("x", "y", "reduced_cost"):
+            assert np.array_equal(getattr(r, f), getattr(w, f)), (i, f)
