@@ -1123,6 +1123,7 @@ enum Slot {
   S_FPE0_NY, S_FPE0_I, S_FPE0_NX,                // post-restart fixed-point error terms
   S_SETUP0, S_SETUP1,                            // setup reductions
   S_LINF_P, S_LINF_D,                            // per_constraint_residual maxima
+  S_OPTIMAL,                                     // a small block's own verdict on its check
   S_COUNT
 };
 
@@ -1814,7 +1815,7 @@ void PdlpSolver<V>::launch_small(long long k, int count, long long limit, bool r
                           ybar_.get(), StepScalars{tau_, sigma_, kr_, 0}, refine_active_, k, count,
                           (int)std::min<long long>(limit, count), restarted, tol.ap + tol.rp * b_norm_,
                           tol.ad + tol.rd * c_norm_, tol.ag, tol.rg, obj_sf_, obj_off_, kkt_point(), kkt_rows(),
-                          kkt_cols(), h_checks_, S_COUNT, S_KKT_RP2, S_KKT_RD2, S_FPE_NY, S_FPE0_NY,
+                          kkt_cols(), h_checks_, S_COUNT, S_KKT_RP2, S_KKT_RD2, S_FPE_NY, S_FPE0_NY, S_OPTIMAL,
                           reinterpret_cast<int*>(h_checks_ + kSmallChecks * S_COUNT)};
   const unsigned lds = (unsigned)small_lds_bytes<V>(m_, n_);
   if (small_ == 1)
@@ -2342,7 +2343,10 @@ int PdlpSolver<V>::pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine)
       fpe = std::sqrt((h_scal_[S_FPE_NX] * omega_ + h_scal_[S_FPE_NY] / omega_) + 2.0 * h_scal_[S_FPE_I] * eta_);
     const size_t rec = R.trace.size();
     R.trace.insert(R.trace.end(), {(double)(k0 + k), l2p_, l2d_, pobj_, dobj_, gap_, 0.0, omega_, fpe, (double)kr_});
-    if (k > 1 && is_optimal(tol)) return done(CUOPT_TERIMINATION_STATUS_OPTIMAL);
+    // A small block has run on past its checks by its own verdict, so that one counts: the
+    // point that is returned is always that of the check that ended the launch.
+    if (k > 1 && (small_ ? h_scal_[S_OPTIMAL] != 0.0 : is_optimal(tol)))
+      return done(CUOPT_TERIMINATION_STATUS_OPTIMAL);
     // first_primal_feasible (pdlp.cu:928-983): a primal feasible, not optimal iterate ends the solve
     if (k > 1 && st_.first_primal_feasible && !bench && primal_feasible(tol))
       return done(CUOPT_TERIMINATION_STATUS_PRIMAL_FEASIBLE);

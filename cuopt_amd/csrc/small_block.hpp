@@ -79,7 +79,7 @@ struct SmallStream {
 
 // All rows of one matrix.  HELD: S holds the stream; otherwise each tile's is loaded
 // here, one round ahead.  Reductions go to part[tile * NRED + k], a sum per tile as
-// tiled_spmv_kernel leaves them.  Ends with a barrier.
+// tiled_spmv_kernel leaves them.  Ends with a barrier (a matrix has a tile at least).
 template <class Epi, int R, bool HELD>
 __device__ inline void small_pass(const SmallShape& M, const int* __restrict__ idx,
                                   const typename Epi::Mat* __restrict__ vals, SmallStream<typename Epi::Mat, R>& S,
@@ -206,6 +206,7 @@ struct SmallArgs {
   KktColsEpi<V> cols;
   double* out;  // kSmallChecks scalar records of `slots` values (host memory), one per check
   int slots, s_rows, s_cols, s_fpe, s_fpe0;  // slots of the sums of the two passes and of the fixed-point error terms
+  int s_optimal;  // and of the verdict on the check
   int* checks;  // number of checks made (host memory)
 };
 
@@ -320,6 +321,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_block_kernel(SmallArgs<V>
       }
       const bool optimal = sqrt(sums[3]) <= A.tol_d && sqrt(sums[0]) <= A.tol_p &&
                            fabs(po - du) <= A.abs_gap + A.rel_gap * (fabs(po) + fabs(du));
+      if (tid == 0) out[A.s_optimal] = optimal ? 1.0 : 0.0;
       if (s == A.count || (k0 > 1 && optimal) || s >= A.limit) break;
     }
     const long long k1 = k0 + 1, k2 = k1 + 1;

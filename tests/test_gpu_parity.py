@@ -1030,3 +1030,40 @@ def test_batch_larger_than_the_free_memory_is_solved_in_parts(prec):
         assert (r.status, r.iterations) == (w.status, w.iterations), i
         for f in ("x", "y", "reduced_cost"):
             assert np.array_equal(getattr(r, f), getattr(w, f)), (i, f)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32_mixed"])
+def test_small_lp_stops_at_the_check_that_meets_the_tolerance_exactly(monkeypatch, prec):
+    # The kernel of a small LP makes its checks itself.  With an absolute tolerance that is
+    # the residual of a check between restart tests, to the last bit, the solve ends at
+    # that check with that check's point; with the next smaller number it runs on.  As the
+    # launches of one check each do.
+    lp = G.random_lp(m=120, n=300, seed=11)
+    # scaled so that only the primal residual is ever above the largest tolerance (0.1)
+    lp = dataclasses.replace(lp, c=1e-6 * lp.c, con_lb=1e-3 * lp.con_lb, con_ub=1e-3 * lp.con_ub,
+                             var_ub=1e-3 * lp.var_ub)
+    prob = c_api.Problem(lp)
+
+    def solve(small, tol=None, limit=400):
+        monkeypatch.setenv("CUOPT_AMD_SMALL", small)
+        conf = c_api.make_settings(0.0, prec, limit, 60.0)
+        if tol is not None:
+            for name, v in (("primal", tol), ("dual", 0.1), ("gap", 0.1)):
+                c_api._check(conf.set(f"absolute_{name}_tolerance", float(v)))
+        return c_api.solve_problem(prob, conf)
+
+    trace = solve("1", limit=200).trace
+    l2p, at = trace[:, 1], trace[:, 0]
+    falls = [i for i in range(3, len(at) - 2) if l2p[i] < l2p[1:i].min() and at[i] % 200]
+    assert len(falls) > 1
+    for i in (falls[0], falls[-1]):
+        at_limit = solve("0", limit=int(at[i]))
+        for tol, ends in ((l2p[i], True), (np.nextafter(l2p[i], 0.0), False)):
+            a, b = solve("0", tol), solve("1", tol)
+            assert (a.status, a.iterations) == (b.status, b.iterations)
+            assert (b.iterations == at[i]) == ends
+            for f in ("x", "y", "reduced_cost", "trace"):  # (the trace's fixed-point error starts as NaN)
+                assert np.array_equal(getattr(a, f), getattr(b, f), equal_nan=True), f
+            if ends:
+                assert b.status == 1 and b.info["l2_primal_residual"] == l2p[i]
+                assert np.array_equal(b.x, at_limit.x) and np.array_equal(b.y, at_limit.y)
