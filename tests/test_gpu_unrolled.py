@@ -506,3 +506,31 @@ def test_more_columns_than_24_bits_number(monkeypatch, prec):
             assert np.array_equal(u, v), (shape, name)
     del many
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("shape,prec,tol", [(s, "fp64", 1e-9) for s in (41, 81, 161, 82)] +
+                         [(s, "fp32_mixed", 2e-3) for s in (41, 81, 161, 82, 84)])
+def test_slab_shapes_match_oracle(monkeypatch, shape, prec, tol):
+    # Every shape of the SpMM kernels (10 x lanes per row + members per lane; 84 is FP32 only)
+    # against the oracle on a ragged matrix, with batches whose last slab is whole, holds
+    # one member and holds some.
+    monkeypatch.setenv("CUOPT_AMD_UNR_SHAPE", str(shape))
+    lp, A = ragged_lp()
+    K, every, lam = 40, 7, 1e-3
+    op = UnrolledPDHG(lp, ridge=lam, steps=K, checkpoint_every=every, precision=prec)
+    b, eta = lp.con_lb.copy(), op.step_size
+    for B in (32, 33, 39):
+        print(f"slab shape {shape} {prec} B={B}", flush=True)
+        rng = np.random.default_rng(shape + B)
+        c = lp.c[None, :] + 0.1 * rng.normal(size=(B, lp.n))
+        ct, bt = (torch.tensor(v, device=DEV, requires_grad=True) for v in (c, b))
+        x, y = op(ct, bt)
+        xo, yo, xs, ys = U.forward(A, c.T.copy(), b, b, lp.var_lb, lp.var_ub, lam, eta, K, keep=True)
+        assert relerr(x.detach().cpu().numpy().T, xo) < tol
+        assert relerr(y.detach().cpu().numpy().T, yo) < tol
+        gx, gy = rng.normal(size=(B, lp.n)), rng.normal(size=(B, lp.m))
+        torch.autograd.backward([x, y], [torch.tensor(v, device=DEV) for v in (gx, gy)])
+        if prec == "fp64":  # (in FP32 a clamp that ends on its other side changes the derivative there)
+            gc, glc, guc = U.backward(A, b, b, lp.var_lb, lp.var_ub, lam, eta, xs, ys, gx.T.copy(), gy.T.copy())
+            assert relerr(ct.grad.cpu().numpy().T, gc) < tol
+            assert relerr(bt.grad.cpu().numpy(), (glc + guc).sum(axis=1)) < tol
