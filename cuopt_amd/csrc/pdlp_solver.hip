@@ -1123,7 +1123,6 @@ enum Slot {
   S_FPE0_NY, S_FPE0_I, S_FPE0_NX,                // post-restart fixed-point error terms
   S_SETUP0, S_SETUP1,                            // setup reductions
   S_LINF_P, S_LINF_D,                            // per_constraint_residual maxima
-  S_OPTIMAL,                                     // a small block's own verdict on its check
   S_COUNT
 };
 
@@ -1289,8 +1288,9 @@ class PdlpSolver {
   hipEvent_t* ev_ = nullptr;  // events of the current timed iteration (benchmark window)
   bool use_graphs_ = true;
   int small_       = 0;      // rounds of the one-workgroup blocks (small_block.hpp); 0: tiled launches
-  double* h_checks_ = nullptr;  // their records, one per check, and the number of checks
+  double* h_checks_ = nullptr;  // their records, one per check, then the number of checks and the last one's verdict
   int checks_made_ = 0, checks_read_ = 0;
+  bool small_optimal_ = false;  // the last of them meets the tolerances
   std::map<std::string, hipGraphExec_t> graphs_;  // captured iteration blocks by pattern
 
   // recentring: the FP64 point (x*, y*), A x*, A^T y*, dual kinks
@@ -1815,7 +1815,7 @@ void PdlpSolver<V>::launch_small(long long k, int count, long long limit, bool r
                           ybar_.get(), StepScalars{tau_, sigma_, kr_, 0}, refine_active_, k, count,
                           (int)std::min<long long>(limit, count), restarted, tol.ap + tol.rp * b_norm_,
                           tol.ad + tol.rd * c_norm_, tol.ag, tol.rg, obj_sf_, obj_off_, kkt_point(), kkt_rows(),
-                          kkt_cols(), h_checks_, S_COUNT, S_KKT_RP2, S_KKT_RD2, S_FPE_NY, S_FPE0_NY, S_OPTIMAL,
+                          kkt_cols(), h_checks_, S_COUNT, S_KKT_RP2, S_KKT_RD2, S_FPE_NY, S_FPE0_NY,
                           reinterpret_cast<int*>(h_checks_ + kSmallChecks * S_COUNT)};
   const unsigned lds = (unsigned)small_lds_bytes<V>(m_, n_);
   if (small_ == 1)
@@ -1824,8 +1824,10 @@ void PdlpSolver<V>::launch_small(long long k, int count, long long limit, bool r
     hipLaunchKernelGGL((small_block_kernel<V, kSmallRounds>), dim3(1), dim3(kSmallThreads), lds, stream_, args);
   CUOPT_HIP_CHECK(hipGetLastError());
   CUOPT_HIP_CHECK(hipStreamSynchronize(stream_));
-  checks_made_ = *reinterpret_cast<const int*>(h_checks_ + kSmallChecks * S_COUNT);
-  checks_read_ = 0;
+  const int* made = reinterpret_cast<const int*>(h_checks_ + kSmallChecks * S_COUNT);
+  checks_made_    = made[0];
+  small_optimal_  = made[1] != 0;
+  checks_read_    = 0;
 }
 
 template <typename V>
@@ -2343,9 +2345,9 @@ int PdlpSolver<V>::pdhg_loop(SolveResult& R, const Tolerances& tol, bool refine)
       fpe = std::sqrt((h_scal_[S_FPE_NX] * omega_ + h_scal_[S_FPE_NY] / omega_) + 2.0 * h_scal_[S_FPE_I] * eta_);
     const size_t rec = R.trace.size();
     R.trace.insert(R.trace.end(), {(double)(k0 + k), l2p_, l2d_, pobj_, dobj_, gap_, 0.0, omega_, fpe, (double)kr_});
-    // A small block has run on past its checks by its own verdict, so that one counts: the
+    // A small block runs on past its checks by its own verdict, so that one counts: the
     // point that is returned is always that of the check that ended the launch.
-    if (k > 1 && (small_ ? h_scal_[S_OPTIMAL] != 0.0 : is_optimal(tol)))
+    if (k > 1 && (small_ ? checks_read_ == checks_made_ && small_optimal_ : is_optimal(tol)))
       return done(CUOPT_TERIMINATION_STATUS_OPTIMAL);
     // first_primal_feasible (pdlp.cu:928-983): a primal feasible, not optimal iterate ends the solve
     if (k > 1 && st_.first_primal_feasible && !bench && primal_feasible(tol))

@@ -206,8 +206,7 @@ struct SmallArgs {
   KktColsEpi<V> cols;
   double* out;  // kSmallChecks scalar records of `slots` values (host memory), one per check
   int slots, s_rows, s_cols, s_fpe, s_fpe0;  // slots of the sums of the two passes and of the fixed-point error terms
-  int s_optimal;  // and of the verdict on the check
-  int* checks;  // number of checks made (host memory)
+  int* checks;  // number of checks made, and whether the last one is optimal (host memory)
 };
 
 // Checks in one launch, at most: the restart test, which the host makes, comes every 200
@@ -295,7 +294,8 @@ __global__ __launch_bounds__(kSmallThreads) void small_block_kernel(SmallArgs<V>
   st.load(MT, A.tidx, A.tw);
   __syncthreads();
   double* const prod64 = reinterpret_cast<double*>(prod_base);
-  int checks = 0;
+  int checks   = 0;
+  bool optimal = false;
   for (int s = 0;; ++s) {
     const long long k0 = A.k + s;  // iterations done
     if (s == A.count || (s > 0 && k0 % small_cond_major(k0) == 0)) {
@@ -319,9 +319,8 @@ __global__ __launch_bounds__(kSmallThreads) void small_block_kernel(SmallArgs<V>
         po = A.obj_sf * (po + A.obj_off);
         du = A.obj_sf * (du + A.obj_off);
       }
-      const bool optimal = sqrt(sums[3]) <= A.tol_d && sqrt(sums[0]) <= A.tol_p &&
-                           fabs(po - du) <= A.abs_gap + A.rel_gap * (fabs(po) + fabs(du));
-      if (tid == 0) out[A.s_optimal] = optimal ? 1.0 : 0.0;
+      optimal = sqrt(sums[3]) <= A.tol_d && sqrt(sums[0]) <= A.tol_p &&
+                fabs(po - du) <= A.abs_gap + A.rel_gap * (fabs(po) + fabs(du));
       if (s == A.count || (k0 > 1 && optimal) || s >= A.limit) break;
     }
     const long long k1 = k0 + 1, k2 = k1 + 1;
@@ -365,7 +364,10 @@ __global__ __launch_bounds__(kSmallThreads) void small_block_kernel(SmallArgs<V>
   }
   for (int j = tid; j < n; j += kSmallThreads) A.x[j] = x[j];
   for (int i = tid; i < m; i += kSmallThreads) A.y[i] = y[i];
-  if (tid == 0) *A.checks = checks;
+  if (tid == 0) {
+    A.checks[0] = checks;
+    A.checks[1] = optimal;
+  }
 }
 
 // ---- power iteration (FP64) ---------------------------------------------------
