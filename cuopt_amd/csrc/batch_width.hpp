@@ -3,8 +3,6 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <functional>
-#include <queue>
 #include <vector>
 
 namespace cuopt_amd {
@@ -28,25 +26,31 @@ inline bool gains_from_width(int nnz, int narrow_blocks) { return nnz >= 2000 &&
 // mean and a few at twice it (u in [0, 1) by reversing the bits of the position).
 inline double batch_launch_time(const std::vector<BatchLp>& lps, size_t nwide, int cus, bool fp32)
 {
-  std::priority_queue<double, std::vector<double>, std::greater<double>> cu, half;
-  for (int i = 0; i < cus; ++i) cu.push(0.0);
+  std::vector<double> free_at(cus, 0.0);  // a heap, the first to be free on top
   double end  = 0.0;
-  auto run_on = [&](auto& free_at, size_t i, double step) {
-    uint32_t r = 0;
-    for (uint32_t v = (uint32_t)i + 1, b = 0; b < 32; ++b, v >>= 1) r = r << 1 | (v & 1);
+  auto run_on = [&](size_t i, double step) {
+    uint32_t r = (uint32_t)i + 1;
+    r = (r & 0x55555555u) << 1 | (r >> 1 & 0x55555555u);
+    r = (r & 0x33333333u) << 2 | (r >> 2 & 0x33333333u);
+    r = (r & 0x0f0f0f0fu) << 4 | (r >> 4 & 0x0f0f0f0fu);
+    r = r << 24 | (r & 0xff00u) << 8 | (r >> 8 & 0xff00u) | r >> 24;
     const double u = r * 0x1p-32, steps = fp32 ? 0.8 + 1.3 * u * u * u : 0.65 + 1.6 * u * u * u * u * u;
-    const double t = free_at.top() + step * steps;
-    free_at.pop();
-    free_at.push(t);
-    end = std::max(end, t);
+    const double t = free_at[0] + step * steps;
+    end            = std::max(end, t);
+    size_t at      = 0;
+    for (size_t c; (c = 2 * at + 1) < free_at.size(); at = c) {  // t in place of the top, sifted down
+      if (c + 1 < free_at.size() && free_at[c + 1] < free_at[c]) ++c;
+      if (free_at[c] >= t) break;
+      free_at[at] = free_at[c];
+    }
+    free_at[at] = t;
   };
   size_t i = 0;
-  for (; i < nwide; ++i) run_on(cu, i, fp32 ? 2.8 + 2.8 * lps[i].wide : 3.1 + 2.45 * lps[i].wide);
-  for (; !cu.empty(); cu.pop()) {
-    half.push(cu.top());
-    half.push(cu.top());
-  }
-  for (; i < lps.size(); ++i) run_on(half, i, (fp32 ? 1.4 : 2.3) + 2.4 * lps[i].narrow);
+  for (; i < nwide; ++i) run_on(i, fp32 ? 2.8 + 2.8 * lps[i].wide : 3.1 + 2.45 * lps[i].wide);
+  std::sort(free_at.begin(), free_at.end());  // halves of the CUs, in order: a heap as well
+  free_at.resize(2 * cus);
+  for (int c = 2 * cus; c-- > 0;) free_at[c] = free_at[c / 2];
+  for (; i < lps.size(); ++i) run_on(i, (fp32 ? 1.4 : 2.3) + 2.4 * lps[i].narrow);
   return end;
 }
 
