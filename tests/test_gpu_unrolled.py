@@ -534,3 +534,43 @@ def test_slab_shapes_match_oracle(monkeypatch, shape, prec, tol):
             gc, glc, guc = U.backward(A, b, b, lp.var_lb, lp.var_ub, lam, eta, xs, ys, gx.T.copy(), gy.T.copy())
             assert relerr(ct.grad.cpu().numpy().T, gc) < tol
             assert relerr(bt.grad.cpu().numpy(), (glc + guc).sum(axis=1)) < tol
+
+
+@pytest.mark.parametrize("most,prec,tol", [(2, "fp64", 1e-9), (4, "fp64", 1e-9), (4, "fp32_mixed", 2e-3)])
+def test_short_rows_match_oracle(monkeypatch, most, prec, tol):
+    # Matrices whose rows (and for the transposed LP columns) have at most two or four nonzeros
+    # take kernels of their own: 0 to `most` nonzeros in a row, every slab shape.
+    import scipy.sparse as sp
+
+    rng = np.random.default_rng(13)
+    rows, cols = 170, 230
+    per = rng.integers(0, most + 1, size=rows)
+    per[:3] = 0, most, 1
+    idx = [np.sort(rng.choice(cols, size=k, replace=False)) for k in per]
+    M = sp.csr_matrix((rng.normal(size=per.sum()), np.concatenate(idx), np.concatenate([[0], np.cumsum(per)])),
+                      shape=(rows, cols))
+    K, every, lam = 30, 7, 1e-3
+    for A in (M, M.T.tocsr()):
+        A.sort_indices()
+        m, n = A.shape
+        b = A @ rng.random(n)
+        lp = G.LP(m=m, n=n, row_offsets=A.indptr.astype(np.int32), col_indices=A.indices.astype(np.int32),
+                  values=A.data, c=rng.normal(size=n), con_lb=b, con_ub=b.copy(), var_lb=np.zeros(n),
+                  var_ub=np.full(n, 10.0))
+        op = UnrolledPDHG(lp, ridge=lam, steps=K, checkpoint_every=every, precision=prec)
+        eta = op.step_size
+        for shape, B in ((0, 1), (0, 3), (0, 40), (41, 6), (81, 11), (161, 21), (82, 19), (84, 37)):
+            print(f"short rows {most} {prec} {m}x{n} shape {shape} B={B}", flush=True)
+            monkeypatch.setenv("CUOPT_AMD_UNR_SHAPE", str(shape))
+            c = lp.c[None, :] + 0.1 * rng.normal(size=(B, n))
+            ct, bt = (torch.tensor(v, device=DEV, requires_grad=True) for v in (c, b))
+            x, y = op(ct, bt)
+            xo, yo, xs, ys = U.forward(A, c.T.copy(), b, b, lp.var_lb, lp.var_ub, lam, eta, K, keep=True)
+            assert relerr(x.detach().cpu().numpy().T, xo) < tol
+            assert relerr(y.detach().cpu().numpy().T, yo) < tol
+            gx = rng.normal(size=(B, n))
+            (x * torch.tensor(gx, device=DEV)).sum().backward()
+            if prec == "fp64":
+                gc, glc, guc = U.backward(A, b, b, lp.var_lb, lp.var_ub, lam, eta, xs, ys, gx.T.copy())
+                assert relerr(ct.grad.cpu().numpy().T, gc) < tol
+                assert relerr(bt.grad.cpu().numpy(), (glc + guc).sum(axis=1)) < tol
