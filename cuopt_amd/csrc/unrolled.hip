@@ -79,22 +79,26 @@ inline int slab_width(Shape s)
 // of one row per wavefront): 200 x 500, B 1 4.33 / 4.16 (4.40); 1 104 x 2 760, B 1 4.62 / 4.23 (4.95);
 // 2 000 x 5 000, B 2 4.87 / 4.45 (5.57); 5 500 x 13 750, B 4 6.09 / 5.46 (9.84); 8 000 x 20 000, B 1
 // 5.31 / 5.11 (12.2); 12 000 x 30 000, B 1 5.57 / 5.91 (16.5); 20 000 x 50 000, B 1 7.19 / 7.67 (24.9).
-// More members: the least
-// (members computed, those past B included) x (cost per member) among the shapes that
-// leave at least kMinWaves wavefronts (one member per lane always may).  Measured, ms,
-// by shape 8x1 / 16x1 / 8x2 / 8x4 (the kernel of one row per wavefront in brackets):
-//   FP32 20 000 x 50 000, B 64, 500 steps with gradients   76.7 / 63.5 / 61.2 / 56.9  (61.4)
-//   FP32  8 000 x 20 000, B 32, 200 steps with gradients    9.25 / 9.04 / 9.01 / 9.83  (11.1)
-//   FP32  1 000 x  2 500, B 40, 200 steps with gradients    5.00 / 5.04 / 5.84 / 6.71  (5.56)
-//   FP32  2 000 x  5 000, B 16, 200 steps                   1.65 / 1.59 / 1.82 / 2.24  (1.81)
-//   FP64 20 000 x 50 000, B 64, 100 steps with gradients    22.5 / 22.0 / 18.5        (22.0)
-//   FP64 16 000 x 40 000, B 12, 200 steps with gradients    12.9 / 12.5 / 11.2        (21.3)
-//   FP64  5 000 x 12 500, B 24, 200 steps with gradients    7.61 / 9.69 / 8.59        (10.6)
-constexpr long long kMinWaves = 1200;
+// More members: the least of the times of both products, estimated as
+//   (members computed, those past B included) x (nonzeros) x (time of a product),
+// and, beyond that and a launch's 5 us, the longest row's chain of sums, which one lane
+// adds up for each of its members in turn.  Shapes of more than one member per lane must
+// leave min_waves wavefronts.  8x1 costs less where the whole launch is small, above all where
+// the slabs are a multiple of the XCDs.  Measured, 60 steps with gradients, ms, by shape 8x1 /
+// 16x1 / 8x2 / 8x4 (the kernel of one row per wavefront in brackets), * the one taken:
+//   FP32 20 000 x 50 000, B 64               9.45 / 8.16 / 7.62 / 7.06*  (7.59)
+//   FP32  5 000 x 12 500, B 64               3.15 / 3.05 / 3.02* / 3.28  (3.29)
+//   FP32  2 000 x  5 000, B 64               1.83* / 2.04 / 2.17 / 2.44  (2.09)
+//   FP32  2 000 x  5 000, B 16               1.69 / 1.61* / 1.83 / 2.12  (1.85)
+//   FP64 20 000 x 50 000, B 64               13.6 / 13.4 / 11.2*         (13.3)
+//   FP64  2 000 x  5 000, B 64               2.02 / 2.42 / 2.10*         (2.51)
+//   FP64  5 000 x 12 500, B 24               2.43* / 2.89 / 2.54         (3.32)
+//   FP32 skewed 20 000 x 50 000 (a row of 26 155), B 64   269 / 211* / 380 / 608 (470)
+//   FP64 skewed  5 000 x 12 500 (a row of  6 856), B 64   63.6 / 48.1* / 73.7    (68.8)
 constexpr int kFewRows        = 24576;
 
 template <typename V>
-Shape pick_shape(int m, int n, int B)
+Shape pick_shape(int m, int n, long long nnz, int alongest, int tlongest, int B)
 {
   if (const char* e = std::getenv("CUOPT_AMD_UNR_SHAPE")) {  // 10 x lanes + members per lane, for tests
     const int v = std::atoi(e);
@@ -103,21 +107,30 @@ Shape pick_shape(int m, int n, int B)
         return s == Shape::k8x4 && sizeof(V) == 8 ? Shape::k8x2 : s;
   }
   if (B <= 4) return std::max(m, n) <= kFewRows ? Shape::k8x1 : Shape::k4x1;
-  Shape best  = Shape::k4x1;
-  double cost = 1e300;
+  constexpr bool kF32 = sizeof(V) == 4;
   struct Option {
     Shape s;
-    int vw;
-    double per_member;
+    int vw, min_waves;
+    double product, chain;  // a product's time against 16x1's, a step of a row's chain in us
   };
-  for (const Option& o : {Option{Shape::k8x1, 1, 1.15}, Option{Shape::k16x1, 1, 1.0}, Option{Shape::k8x2, 2, 0.95},
-                          Option{Shape::k8x4, 4, 0.9}}) {
-    const long long W = slab_width(o.s), members = (B + W - 1) / W * W;
+  const Option options[] = {{Shape::k8x1, 1, 0, kF32 ? 1.15 : 1.1, kF32 ? 0.055 : 0.050},
+                            {Shape::k16x1, 1, 0, 1.0, kF32 ? 0.043 : 0.036},
+                            {Shape::k8x2, 2, kF32 ? 1200 : 500, kF32 ? 0.95 : 0.85, kF32 ? 0.076 : 0.060},
+                            {Shape::k8x4, 4, 1500, 0.9, 0.120}};
+  Shape best  = Shape::k4x1;
+  double cost = 1e300;
+  for (const Option& o : options) {
+    const long long W = slab_width(o.s), slabs = (B + W - 1) / W, members = slabs * W;
     if (o.vw * sizeof(V) > 16) continue;
-    if (o.vw > 1 && (long long)std::min(m, n) * members / (kWave * o.vw) < kMinWaves) continue;
+    if (std::min(m, n) * members / (kWave * o.vw) < o.min_waves) continue;
     if ((unsigned long long)std::max(m, n) * W * sizeof(V) >= (1ULL << 32)) continue;  // 32-bit gather offsets
-    if (members * o.per_member < cost) {
-      cost = members * o.per_member;
+    double product = o.product;
+    if (o.s == Shape::k8x1 && members * nnz < 3000000) product = slabs % kXcds == 0 ? 0.95 : 1.02;
+    const double us = (kF32 ? 0.8e-6 : 1.2e-6) * product * members * nnz;  // one launch
+    double both     = 2.0 * us;
+    for (int longest : {alongest, tlongest}) both += std::max(0.0, o.chain * longest - std::max(us, 5.0));
+    if (both < cost) {
+      cost = both;
       best = o.s;
     }
   }
@@ -753,7 +766,7 @@ struct UnrolledImpl {
 template <typename V>
 Shape pick_shape(const UnrolledImpl& U, int B)
 {
-  return pick_shape<V>(U.m, U.n, B);
+  return pick_shape<V>(U.m, U.n, U.nnz, U.alongest, U.tlongest, B);
 }
 
 // Graph replay of full segments unless CUOPT_AMD_GRAPHS=0 (direct launches of
