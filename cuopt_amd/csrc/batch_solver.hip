@@ -500,9 +500,9 @@ struct BScaleEpi {
 };
 
 // One product of the power iteration or Lanczos over a scaled FP64 matrix: A~^T q, or
-// A~ (A~^T q) with the power iteration's q . (A~ A~^T q).  `vec` is gathered (through
-// LdsGather or GlobalGather, which read it through a typed pointer), out is one
-// value per row; both are LDS or global memory, by LP.  Each step was bound by its
+// A~ (A~^T q) with the power iteration's q . (A~ A~^T q).  The gathered vector and `out`,
+// one value per row, are LDS or global memory, by LP; rows_pass gathers through what
+// it is given (LdsGather or GlobalGather, a typed pointer).  Each step was bound by its
 // gathers: forming ((a D_r) D_c) (z / ||z||) per nonzero took two gathers and an FP64
 // division; reading the scaled values that the loop uses anyway (and a copy of them
 // in FP64 for FP32-mixed), with z / ||z|| formed once per row, leaves one gather.

@@ -95,7 +95,7 @@ inline int slab_width(Shape s)
 //   FP64  5 000 x 12 500, B 24               2.43* / 2.89 / 2.54         (3.32)
 //   FP32 skewed 20 000 x 50 000 (a row of 26 155), B 64   269 / 211* / 380 / 608 (470)
 //   FP64 skewed  5 000 x 12 500 (a row of  6 856), B 64   63.6 / 48.1* / 73.7    (68.8)
-constexpr int kFewRows        = 24576;
+constexpr int kFewRows = 24576;
 
 template <typename V>
 Shape pick_shape(int m, int n, long long nnz, int alongest, int tlongest, int B)
@@ -318,11 +318,12 @@ __device__ inline double group_value(double v)
 // more) are issued before its sums, and the next chunk's indices and values in
 // between.
 //
-// In FP32 these kernels are bound by the vector ALU (87 % busy: ten operations per
-// product for the compensated sum), so the rest is kept small: a gather is one 32-bit
-// offset from a scalar base (slabs of 4 members, which also serve matrices whose
-// wider slabs would pass 4 GiB, take 64 bits), and a chunk that is whole in every row
-// of the wavefront is summed without looking at the rows' ends.
+// In FP32 the vector ALU is what bounds the forward steps (at 20 000 x 50 000, B = 64 it
+// issues in 81-84 % of the CUs' busy cycles; ten operations per product for the compensated
+// sum), and most of the adjoint steps' time (58-66 %; they also read and write more).  So the
+// rest is kept small: a gather is one 32-bit offset from a scalar base (64 bits only where a
+// slab's operand needs them, BIG), and a chunk that is whole in every row of the wavefront
+// is summed without looking at the rows' ends.
 template <typename V, class L, int... I>
 __device__ inline void row_dot_chunks(const MatView<V>& M, const Place& p, const V* __restrict__ slab,
                                       typename AccFor<V>::type (&a)[L::VW], std::integer_sequence<int, I...>)
