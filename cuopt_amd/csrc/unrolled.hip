@@ -54,7 +54,7 @@ constexpr unsigned kXcds = 8;    // the XCDs, which take the workgroups of a lau
 //
 // Gathers of W contiguous values use the lanes that a wavefront per row leaves idle below
 // 64 members, and a slab's operand is smaller than the whole: at 20 000 x 50 000 and
-// B = 64 in FP32 slabs of 32 cut the dual step's L2 misses from 733 k to 592 k lines.
+// B = 64 in FP32 slabs of 32 cut the dual step's L2 misses from 733 k to 607 k lines.
 template <int LW_, int VW_, bool BIG_, int SHORT_>
 struct Lanes {
   static constexpr int LW = LW_;             // lanes per row
